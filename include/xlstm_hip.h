@@ -283,6 +283,30 @@ int xl_gate_proj_softcap_fwd(const void* x, const void* weight, const void* bias
                              int M, int D, int G, float cap, int cap_rounding, int dtype, void* stream);
 
 /*
+ * Two gate projections over the same rows, without stacking their weights: y1 [M, G1] and y2 [M, G2] as
+ * xl_gate_proj_softcap_fwd computes them from w1 [G1, D], bias1 and w2 [G2, D], bias2 (G1 + G2 <= 64).
+ * tokens_per_seq > 0: row m = b * tokens_per_seq + s, outputs head-major, y1 [B, G1, tokens_per_seq]
+ * (the chunkwise kernels' gate layout); 0: token-major.
+ */
+int xl_gate_proj2_softcap_fwd(const void* x, const void* w1, const void* bias1, int G1, const void* w2,
+                              const void* bias2, int G2, void* y1, void* y2, int M, int D, int tokens_per_seq,
+                              float cap, int cap_rounding, int dtype, void* stream);
+
+/*
+ * sum = x + residual (rounded to the dtype; residual NULL: sum not written, x itself) and
+ * y = sum / sqrt(mean(sum^2) + eps) * weight per row of [M, D], float32, rounded once: a block's
+ * residual add and the RMSNorm after it (xlstm_metal/torch_native/blocks/mlstm/mlstm_block.py:163-206).
+ * copy_*: up to two float32 buffers copied along.  bf16 / f16, D a multiple of 8, 16-byte aligned.
+ */
+int xl_add_rmsnorm_fwd(const void* x, const void* residual, const void* weight, void* sum, void* y, int M, int D,
+                       float eps, const float* copy_src0, float* copy_dst0, int ncopy0, const float* copy_src1,
+                       float* copy_dst1, int ncopy1, int dtype, void* stream);
+
+/* y = silu(gate) * up, the SiLU rounded to the dtype first (the SwiGLU FFN's product).  bf16 / f16,
+ * numel a multiple of 8, 16-byte aligned. */
+int xl_silu_mul_fwd(const void* gate, const void* up, void* y, int64_t numel, int dtype, void* stream);
+
+/*
  * Chunkwise mLSTM backward: the reference's custom backward mlstm_chunkwise_bw
  * (kernel_development/xlstm/mlstm_block/mlstm_chunkwise/vendored/torch/native/
  * bw.py:198-352, wrapped by _mlstm_chunkwise_fwbw.backward, fwbw.py:102-173 and

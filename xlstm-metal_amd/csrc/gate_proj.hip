@@ -58,6 +58,41 @@ __device__ __forceinline__ float gate_epilogue(float acc, float bn, float cap, f
   return v;
 }
 
+// One or two weight matrices over the same rows: output n < G1 from w, n >= G1 from w2 (row n - G1),
+// each with its bias (or null) and its own output.  seq > 0: outputs head-major, [B, G, seq], row
+// m = b * seq + s (what the chunkwise kernels read; the token-major form needed a strided copy per
+// gate); 0: token-major [M, G].
+template <typename T>
+struct GateOut {
+  const T* w;
+  const T* w2;
+  const T* bias;
+  const T* bias2;
+  T* y;
+  T* y2;
+  int G1, G, seq;
+  __device__ __forceinline__ const T* wrow(int n, int D) const {
+    return n < G1 ? w + (size_t)n * D : w2 + (size_t)(n - G1) * D;
+  }
+  __device__ __forceinline__ float bias_of(int n) const {
+    const T* b = n < G1 ? bias : bias2;
+    return b ? to_f32(b[n < G1 ? n : n - G1]) : 0.0f;
+  }
+  __device__ __forceinline__ void store(int m, int n, float v) const {
+    const bool first = n < G1;
+    T* out = first ? y : y2;
+    const int c = first ? n : n - G1, g = first ? G1 : G - G1;
+    size_t at;
+    if (seq > 0) {
+      const int b = m / seq;
+      at = ((size_t)b * g + c) * seq + (m - b * seq);
+    } else {
+      at = (size_t)m * g + c;
+    }
+    out[at] = from_f32<T>(v);
+  }
+};
+
 constexpr int GP_WAVES = 4;  // waves per 16-row tile, each over a quarter of the k-steps
 constexpr int GP_BLOCK = 64 * GP_WAVES;
 
@@ -65,10 +100,8 @@ constexpr int GP_BLOCK = 64 * GP_WAVES;
 // contiguous ranges (4x the loads in flight of one wave per tile) and their
 // partial 16 x 16 accumulators are summed through LDS by wave 0.
 template <typename T, int NT>
-__global__ __launch_bounds__(GP_BLOCK) void gate_proj_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                             const T* __restrict__ bias, T* __restrict__ y, int M,
-                                                             int D, int G, float cap, float inv_cap,
-                                                             int cap_rounding) {
+__global__ __launch_bounds__(GP_BLOCK) void gate_proj_kernel(const T* __restrict__ x, GateOut<T> o, int M, int D,
+                                                             float cap, float inv_cap, int cap_rounding) {
   __shared__ f32x4 s_part[GP_WAVES - 1][NT][64];
   const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15, wv = threadIdx.x >> 6;
   const int m0 = blockIdx.x * 16;
@@ -80,7 +113,7 @@ __global__ __launch_bounds__(GP_BLOCK) void gate_proj_kernel(const T* __restrict
   // weight rows past G re-read row G - 1 (their columns are not stored)
   const T* wr[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) wr[nt] = w + (size_t)min(nt * 16 + r16, G - 1) * D + 8 * g;
+  for (int nt = 0; nt < NT; ++nt) wr[nt] = o.wrow(min(nt * 16 + r16, o.G - 1), D) + 8 * g;
 
   // k-slice [32 ks + 8 g, +8) of a row lies wholly inside or outside D (D % 8 == 0);
   // past D (or past this wave's range) the address is clamped in bounds and both
@@ -153,29 +186,27 @@ __global__ __launch_bounds__(GP_BLOCK) void gate_proj_kernel(const T* __restrict
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int n = nt * 16 + r16;
-    if (n >= G) continue;
-    const float bn = bias ? to_f32(bias[n]) : 0.0f;
+    if (n >= o.G) continue;
+    const float bn = o.bias_of(n);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int m = m0 + 4 * g + e;
       if (m >= M) continue;
-      y[(size_t)m * G + n] = from_f32<T>(gate_epilogue<T>(acc[nt][e], bn, cap, inv_cap, cap_rounding));
+      o.store(m, n, gate_epilogue<T>(acc[nt][e], bn, cap, inv_cap, cap_rounding));
     }
   }
 }
 
 // Row form: X streamed row by row, the G weight rows as the small rows; lane n < G of the wave
-// ends each row with output n, stored as one contiguous row of y.
+// ends each row with output n.
 template <typename T, int MT, int NPC>
-__global__ __launch_bounds__(64 * rowgemv::WAVES) void gate_rows_kernel(const T* __restrict__ x,
-                                                                        const T* __restrict__ w,
-                                                                        const T* __restrict__ bias,
-                                                                        T* __restrict__ y, int M, int D, int G,
-                                                                        float cap, float inv_cap, int cap_rounding) {
+__global__ __launch_bounds__(64 * rowgemv::WAVES) void gate_rows_kernel(const T* __restrict__ x, GateOut<T> o, int M,
+                                                                        int D, float cap, float inv_cap,
+                                                                        int cap_rounding) {
   const int lane = threadIdx.x & 63;
-  const float bn = (bias && lane < G) ? to_f32(bias[lane]) : 0.0f;
-  rowgemv::stream_rows<T, MT, NPC>(w, G, x, M, D, [&](int r, int ln, float dot) {
-    if (ln < G) y[(size_t)r * G + ln] = from_f32<T>(gate_epilogue<T>(dot, bn, cap, inv_cap, cap_rounding));
+  const float bn = lane < o.G ? o.bias_of(lane) : 0.0f;
+  rowgemv::stream_rows<T, MT, NPC>(o.w, o.G1, o.w2, o.G, x, M, D, [&](int r, int ln, float dot) {
+    if (ln < o.G) o.store(r, ln, gate_epilogue<T>(dot, bn, cap, inv_cap, cap_rounding));
   });
 }
 
@@ -187,27 +218,49 @@ const void* gate_rows(int G, int D) {
 }
 
 template <typename T>
-int launch(const void* x, const void* w, const void* b, void* y, int M, int D, int G, float cap, int cap_rounding,
-           hipStream_t st) {
+int launch(const char* who, const void* x, const void* w1, const void* b1, int G1, const void* w2, const void* b2, int G2,
+           void* y1, void* y2, int M, int D, int seq, float cap, int cap_rounding, hipStream_t st) {
+  const int G = G1 + G2;
+  float inv_cap = cap > 0.0f ? 1.0f / cap : 0.0f;
+  GateOut<T> o{(const T*)w1, (const T*)w2, (const T*)b1, (const T*)b2, (T*)y1, (T*)y2, G1, G, seq};
   if (const void* rk = gate_rows<T>(G, D)) {
-    const float inv = cap > 0.0f ? 1.0f / cap : 0.0f;
-    void* args[] = {(void*)&x, (void*)&w,   (void*)&b,   (void*)&y,   (void*)&M,
-                    (void*)&D, (void*)&G,   (void*)&cap, (void*)&inv, (void*)&cap_rounding};
-    return rowgemv::launch_streaming(rk, args, M, st, "xl_gate_proj_softcap_fwd");
+    void* args[] = {(void*)&x, (void*)&o, (void*)&M, (void*)&D, (void*)&cap, (void*)&inv_cap, (void*)&cap_rounding};
+    return rowgemv::launch_streaming(rk, args, M, st, who);
   }
   const int64_t blocks = ((int64_t)M + 15) / 16;
-  if (blocks > 0x7fffffff) return set_error(XL_ERR_UNSUPPORTED, "xl_gate_proj_softcap_fwd: M=%d too large", M);
-  const float inv_cap = cap > 0.0f ? 1.0f / cap : 0.0f;
-  const T *xp = (const T*)x, *wp = (const T*)w, *bp = (const T*)b;
-  T* yp = (T*)y;
+  if (blocks > 0x7fffffff) return set_error(XL_ERR_UNSUPPORTED, "%s: M=%d too large", who, M);
+  const T* xp = (const T*)x;
   const dim3 grid((unsigned)blocks), blk(GP_BLOCK);
   switch ((G + 15) / 16) {
-    case 1: hipLaunchKernelGGL((gate_proj_kernel<T, 1>), grid, blk, 0, st, xp, wp, bp, yp, M, D, G, cap, inv_cap, cap_rounding); break;
-    case 2: hipLaunchKernelGGL((gate_proj_kernel<T, 2>), grid, blk, 0, st, xp, wp, bp, yp, M, D, G, cap, inv_cap, cap_rounding); break;
-    case 3: hipLaunchKernelGGL((gate_proj_kernel<T, 3>), grid, blk, 0, st, xp, wp, bp, yp, M, D, G, cap, inv_cap, cap_rounding); break;
-    default: hipLaunchKernelGGL((gate_proj_kernel<T, 4>), grid, blk, 0, st, xp, wp, bp, yp, M, D, G, cap, inv_cap, cap_rounding); break;
+    case 1: hipLaunchKernelGGL((gate_proj_kernel<T, 1>), grid, blk, 0, st, xp, o, M, D, cap, inv_cap, cap_rounding); break;
+    case 2: hipLaunchKernelGGL((gate_proj_kernel<T, 2>), grid, blk, 0, st, xp, o, M, D, cap, inv_cap, cap_rounding); break;
+    case 3: hipLaunchKernelGGL((gate_proj_kernel<T, 3>), grid, blk, 0, st, xp, o, M, D, cap, inv_cap, cap_rounding); break;
+    default: hipLaunchKernelGGL((gate_proj_kernel<T, 4>), grid, blk, 0, st, xp, o, M, D, cap, inv_cap, cap_rounding); break;
   }
-  return check_launch("xl_gate_proj_softcap_fwd");
+  return check_launch(who);
+}
+
+int gate_proj(const char* who, const void* x, const void* w1, const void* b1, int G1, const void* w2, const void* b2,
+              int G2, void* y1, void* y2, int M, int D, int seq, float cap, int cap_rounding, int dtype, hipStream_t st) {
+  const int64_t G = (int64_t)G1 + G2;
+  if (M < 0 || D < 0 || G1 < 0 || G2 < 0 || seq < 0)
+    return set_error(XL_ERR_INVALID_ARG, "%s: negative size (M=%d D=%d G=%lld)", who, M, D, (long long)G);
+  if (!dtype_ok(dtype)) return set_error(XL_ERR_INVALID_ARG, "%s: unknown dtype %d", who, dtype);
+  if (dtype == XL_DTYPE_F32) return set_error(XL_ERR_UNSUPPORTED, "%s: float32 (bf16 / f16 MFMA kernel only)", who);
+  if (G > 64) return set_error(XL_ERR_UNSUPPORTED, "%s: G=%lld outputs (at most 64)", who, (long long)G);
+  if (D % 8 != 0 || (D == 0 && M > 0 && G > 0))
+    return set_error(XL_ERR_UNSUPPORTED, "%s: D=%d (a positive multiple of 8)", who, D);
+  if (!(cap == cap) || cap == INFINITY) return set_error(XL_ERR_INVALID_ARG, "%s: cap must be finite", who);
+  if (cap_rounding != 0 && cap_rounding != 1)
+    return set_error(XL_ERR_INVALID_ARG, "%s: cap_rounding must be 0 or 1", who);
+  if (seq > 0 && M % seq != 0)
+    return set_error(XL_ERR_INVALID_ARG, "%s: M=%d rows are no whole number of %d-token sequences", who, M, seq);
+  if ((int64_t)M * G == 0) return XL_OK;
+  if (!x || (G1 && (!w1 || !y1)) || (G2 && (!w2 || !y2))) return set_error(XL_ERR_INVALID_ARG, "%s: null pointer", who);
+  if ((((uintptr_t)x) | ((uintptr_t)w1) | ((uintptr_t)w2)) & 15u)
+    return set_error(XL_ERR_INVALID_ARG, "%s: x and weight must be 16-byte aligned", who);
+  if (dtype == XL_DTYPE_BF16) return launch<bf16_t>(who, x, w1, b1, G1, w2, b2, G2, y1, y2, M, D, seq, cap, cap_rounding, st);
+  return launch<f16_t>(who, x, w1, b1, G1, w2, b2, G2, y1, y2, M, D, seq, cap, cap_rounding, st);
 }
 
 }  // namespace
@@ -215,24 +268,15 @@ int launch(const void* x, const void* w, const void* b, void* y, int M, int D, i
 
 extern "C" int xl_gate_proj_softcap_fwd(const void* x, const void* weight, const void* bias, void* y, int M, int D,
                                         int G, float cap, int cap_rounding, int dtype, void* stream) {
-  using namespace xl;
-  clear_error();
-  if (M < 0 || D < 0 || G < 0)
-    return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: negative size (M=%d D=%d G=%d)", M, D, G);
-  if (!dtype_ok(dtype)) return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: unknown dtype %d", dtype);
-  if (dtype == XL_DTYPE_F32)
-    return set_error(XL_ERR_UNSUPPORTED, "xl_gate_proj_softcap_fwd: float32 (bf16 / f16 MFMA kernel only)");
-  if (G > 64) return set_error(XL_ERR_UNSUPPORTED, "xl_gate_proj_softcap_fwd: G=%d outputs (at most 64)", G);
-  if (D % 8 != 0 || (D == 0 && M > 0 && G > 0))
-    return set_error(XL_ERR_UNSUPPORTED, "xl_gate_proj_softcap_fwd: D=%d (a positive multiple of 8)", D);
-  if (!(cap == cap) || cap == INFINITY) return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: cap must be finite");
-  if (cap_rounding != 0 && cap_rounding != 1)
-    return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: cap_rounding must be 0 or 1");
-  if ((int64_t)M * G == 0) return XL_OK;
-  if (!x || !weight || !y) return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: null pointer");
-  if ((((uintptr_t)x) | ((uintptr_t)weight)) & 15u)
-    return set_error(XL_ERR_INVALID_ARG, "xl_gate_proj_softcap_fwd: x and weight must be 16-byte aligned");
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == XL_DTYPE_BF16) return launch<bf16_t>(x, weight, bias, y, M, D, G, cap, cap_rounding, st);
-  return launch<f16_t>(x, weight, bias, y, M, D, G, cap, cap_rounding, st);
+  xl::clear_error();
+  return xl::gate_proj("xl_gate_proj_softcap_fwd", x, weight, bias, G, nullptr, nullptr, 0, y, nullptr, M, D, 0, cap,
+                       cap_rounding, dtype, (hipStream_t)stream);
+}
+
+extern "C" int xl_gate_proj2_softcap_fwd(const void* x, const void* w1, const void* bias1, int G1, const void* w2,
+                                         const void* bias2, int G2, void* y1, void* y2, int M, int D, int tokens_per_seq,
+                                         float cap, int cap_rounding, int dtype, void* stream) {
+  xl::clear_error();
+  return xl::gate_proj("xl_gate_proj2_softcap_fwd", x, w1, bias1, G1, w2, bias2, G2, y1, y2, M, D, tokens_per_seq, cap,
+                       cap_rounding, dtype, (hipStream_t)stream);
 }

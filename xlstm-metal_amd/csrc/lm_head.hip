@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64 * rowgemv::WAVES) void lm_head_rows_kernel(const
                                                                            const T* __restrict__ w,
                                                                            T* __restrict__ y, int M, int D, int V,
                                                                            float cap, float inv_cap) {
-  rowgemv::stream_rows<T, MT, NPC>(x, M, w, V, D, [&](int r, int lane, float logit) {
+  rowgemv::stream_rows<T, MT, NPC>(x, M, x, M, w, V, D, [&](int r, int lane, float logit) {
     if (lane < M) {
       float z = round_to<T>(logit);  // the Linear's output in its dtype
       if (cap > 0.0f) z = soft_cap16(z, cap, inv_cap);

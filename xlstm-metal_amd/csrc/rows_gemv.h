@@ -50,10 +50,10 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
 }
 
 // The whole wave calls epi(r, lane, dot) after each streamed row r; lane m < MT
-// holds dot(S[r], X[m]) (0 for m >= M).
+// holds dot(S[r], X[m]) (0 for m >= M).  The small rows are M1 rows of x, then M - M1 rows of x2.
 template <typename T, int MT, int NPC, typename Epi>
-__device__ __forceinline__ void stream_rows(const T* __restrict__ x, int M, const T* __restrict__ s, int R, int D,
-                                            Epi&& epi) {
+__device__ __forceinline__ void stream_rows(const T* __restrict__ x, int M1, const T* __restrict__ x2, int M,
+                                            const T* __restrict__ s, int R, int D, Epi&& epi) {
   const int lane = threadIdx.x & 63;
   const int nw = gridDim.x * WAVES;
   const int gw = blockIdx.x * WAVES + (threadIdx.x >> 6);
@@ -63,7 +63,9 @@ __device__ __forceinline__ void stream_rows(const T* __restrict__ x, int M, cons
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int p = 0; p < NPC; ++p)
-      xr[m][p] = m < M ? *reinterpret_cast<const u32x4*>(x + (size_t)m * D + 512 * p + 8 * lane) : zero;
+      xr[m][p] = m < M ? *reinterpret_cast<const u32x4*>((m < M1 ? x + (size_t)m * D : x2 + (size_t)(m - M1) * D) +
+                                                         512 * p + 8 * lane)
+                       : zero;
   // lane (g, r16) holds D[4g + e][r16], e = 0..3: the diagonal element D[i][i] sits in lane
   // 16 (i >> 2) + i at e = i & 3
   const bool on_diag = (lane >> 4) == ((lane & 15) >> 2);

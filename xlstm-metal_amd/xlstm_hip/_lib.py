@@ -47,6 +47,9 @@ SIGNATURES = {
     "xl_mh_rmsnorm_gate_fwd": (_i, [_vp] * 4 + [_i] * 5 + [_f, _i, _vp]),
     "xl_gate_proj_softcap_fwd": (_i, [_vp] * 4 + [_i] * 3 + [_f, _i, _i, _vp]),
     "xl_lm_head_softcap_fwd": (_i, [_vp] * 3 + [_i] * 3 + [_f, _i, _vp]),
+    "xl_gate_proj2_softcap_fwd": (_i, [_vp] * 3 + [_i, _vp, _vp, _i, _vp, _vp] + [_i] * 3 + [_f, _i, _i, _vp]),
+    "xl_add_rmsnorm_fwd": (_i, [_vp] * 5 + [_i, _i, _f] + [_fp, _fp, _i] * 2 + [_i, _vp]),
+    "xl_silu_mul_fwd": (_i, [_vp] * 3 + [_i64, _i, _vp]),
 }
 
 ABI_VERSION = 2

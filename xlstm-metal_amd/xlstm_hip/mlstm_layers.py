@@ -17,7 +17,7 @@ Drop-ins (paths relative to the reference root, ``TNM`` =
 
 * ``mLSTMProjectionCell`` (``TNM/mlstm_chunkwise/mlstm_projection_cell.py:18-106``): the
   q, k, v projections stay ``nn.Linear``; the two gate projections and their soft-cap are one
-  kernel (``gate_proj_kernel``) over the stacked gate weights.
+  kernel (``gate_proj_kernel``) that reads x once and writes them head-major.
 
 State-dict keys match the reference modules.
 """
@@ -31,10 +31,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
-from .ops import gate_proj_softcap_op, mh_rmsnorm_gate_op
+from .ops import gate_proj2_softcap_op, gate_proj_softcap_op, mh_rmsnorm_gate_op
 from .soft_cap import soft_cap
 
-__all__ = ["mh_rmsnorm_gate", "gate_proj_softcap", "stacked_linears", "MultiHeadRMSNorm", "MultiHeadLayerNorm",
+__all__ = ["mh_rmsnorm_gate", "gate_proj_softcap", "gate_pair_softcap", "stacked_linears", "MultiHeadRMSNorm", "MultiHeadLayerNorm",
            "mLSTMProjectionCell", "mLSTMOutputCell"]
 
 
@@ -64,6 +64,20 @@ def stacked_linears(*linears: nn.Linear):
         return w, None
     b = torch.cat([lin.bias if lin.bias is not None else lin.weight.new_zeros(lin.out_features) for lin in linears])
     return w, b
+
+
+def gate_pair_softcap(x: Tensor, first: nn.Linear, second: nn.Linear, cap: Optional[float] = None,
+                      cap_in_dtype: bool = False, heads_first: bool = False):
+    """``gate_proj_softcap`` of two Linear layers over x [B, S, D]: two outputs [B, S, G], or [B, G, S] with
+    ``heads_first``.  bf16 / f16: one kernel that reads x once and writes either layout (stacking the
+    weights first cost two copies a call, slicing the stacked output two more); float32: the stacked
+    projection."""
+    if x.dtype == torch.float32 or x.dim() != 3:
+        g = gate_proj_softcap(x, *stacked_linears(first, second), cap, cap_in_dtype)
+        g1, g2 = g[..., :first.out_features], g[..., first.out_features:]
+        return (g1.permute(0, 2, 1), g2.permute(0, 2, 1)) if heads_first else (g1, g2)
+    return gate_proj2_softcap_op(x, first.weight, first.bias, second.weight, second.bias,
+                                 0.0 if cap is None else float(cap), 1 if cap_in_dtype else 0, heads_first)
 
 
 def mh_rmsnorm_gate(h: Tensor, weight: Optional[Tensor] = None, o_preact: Optional[Tensor] = None,
@@ -98,7 +112,7 @@ class MultiHeadRMSNorm(nn.Module):
 
 class mLSTMProjectionCell(nn.Module):
     """``mlstm_projection_cell.py:18-106``: q, k, v [B, NH, S, DH] (permuted views) and the soft-capped
-    gate pre-activations i, f [B, NH, S] (permuted views) of x [B, S, input_size]."""
+    gate pre-activations i, f [B, NH, S] of x [B, S, input_size]."""
 
     def __init__(self, input_size: int, num_heads: int, qk_dim_per_head: int, v_dim_per_head: int,
                  use_bias: bool = False, gate_soft_cap: Optional[float] = None) -> None:
@@ -121,8 +135,8 @@ class mLSTMProjectionCell(nn.Module):
         q = self.q_proj(x).view(B, S, NH, self.qk_dim_per_head).permute(0, 2, 1, 3)
         k = self.k_proj(x).view(B, S, NH, self.qk_dim_per_head).permute(0, 2, 1, 3)
         v = self.v_proj(x).view(B, S, NH, self.v_dim_per_head).permute(0, 2, 1, 3)
-        g = gate_proj_softcap(x, *stacked_linears(self.igate_proj, self.fgate_proj), self.gate_soft_cap)
-        return q, k, v, g[..., :NH].permute(0, 2, 1), g[..., NH:].permute(0, 2, 1)
+        i, f = gate_pair_softcap(x, self.igate_proj, self.fgate_proj, self.gate_soft_cap, heads_first=True)
+        return q, k, v, i, f
 
 
 class MultiHeadLayerNorm(nn.Module):

@@ -10,7 +10,7 @@ no CPU path: CPU tensors raise.
 from __future__ import annotations
 
 import warnings
-from typing import Optional
+from typing import List, Optional, Sequence
 
 import torch
 from torch import Tensor
@@ -20,7 +20,8 @@ from . import _lib
 __all__ = [
     "soft_cap_op", "mlstm_step_op", "mlstm_step_inplace_op", "mlstm_chunkwise_op", "mlstm_chunkwise_bwd_op", "mlstm_sequence_op",
     "slstm_step_op", "slstm_sequence_op", "causal_conv1d_op", "group_norm_op", "mh_rmsnorm_gate_op",
-    "gate_proj_softcap_op", "lm_head_softcap_op", "chunkwise_workspace_bytes", "chunkwise_algorithm",
+    "gate_proj_softcap_op", "gate_proj2_softcap_op", "lm_head_softcap_op", "rms_norm_op", "add_rmsnorm_op", "silu_mul_op",
+    "chunkwise_workspace_bytes", "chunkwise_algorithm",
 ]
 
 _EMPTY_SHAPE = (0,)
@@ -571,6 +572,103 @@ def gate_proj_softcap_op(x: Tensor, weight: Tensor, bias: Optional[Tensor], cap:
 @gate_proj_softcap_op.register_fake
 def _(x, weight, bias, cap, cap_rounding=0):
     return x.new_empty(tuple(x.shape[:-1]) + (weight.shape[0],))
+
+
+@torch.library.custom_op("xlstm_hip::gate_proj2_softcap", mutates_args=())
+def gate_proj2_softcap_op(x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor], cap: float,
+                          cap_rounding: int, heads_first: bool) -> tuple[Tensor, Tensor]:
+    """gate_proj_softcap_op for two projections of one input [B, S, D], their weights not stacked; the
+    outputs [B, S, G], or [B, G, S] with ``heads_first``."""
+    what = "gate_proj_softcap"
+    _lib.require_gpu(x, w1, b1, w2, b2, what=what)
+    _check(x.dim() == 3, what, f"x must be (B, S, D), got {tuple(x.shape)}")
+    B, S, D = x.shape
+    for w, b in ((w1, b1), (w2, b2)):
+        _check(w.dim() == 2 and w.shape[1] == D, what,
+               f"weight must be (G, D) with D = x.shape[-1], got {tuple(w.shape)} for x {tuple(x.shape)}")
+        _check(b is None or tuple(b.shape) == (w.shape[0],), what, f"bias must be ({w.shape[0]},)")
+        _check(w.dtype == x.dtype and (b is None or b.dtype == x.dtype), what, "x, weight and bias must share a dtype")
+    x, w1, w2 = _prep(x), _prep(w1), _prep(w2)
+    b1, b2 = (None if b is None else _prep(b) for b in (b1, b2))
+    G1, G2 = w1.shape[0], w2.shape[0]
+    y1, y2 = (torch.empty((B, G, S) if heads_first else (B, S, G), dtype=x.dtype, device=x.device) for G in (G1, G2))
+    rc = _lib.load().xl_gate_proj2_softcap_fwd(
+        x.data_ptr(), w1.data_ptr(), _lib.ptr(b1), G1, w2.data_ptr(), _lib.ptr(b2), G2, y1.data_ptr(), y2.data_ptr(),
+        B * S, D, S if heads_first else 0, float(cap), int(cap_rounding), _lib.dtype_code(x, what), _lib.stream_of(x))
+    _lib.check(rc, what)
+    return y1, y2
+
+
+@gate_proj2_softcap_op.register_fake
+def _(x, w1, b1, w2, b2, cap, cap_rounding, heads_first):
+    B, S, _ = x.shape
+    return tuple(x.new_empty((B, w.shape[0], S) if heads_first else (B, S, w.shape[0])) for w in (w1, w2))
+
+
+# ------------------------------------------- a block's norm (with the residual before it), SwiGLU product
+def _add_rmsnorm(x, r, weight, eps, copy_src, copy_dst, what):
+    _lib.require_gpu(x, r, weight, *copy_src, *copy_dst, what=what)
+    D = x.shape[-1]
+    _check(tuple(weight.shape) == (D,) and weight.dtype == x.dtype, what, f"weight must be ({D},) of {x.dtype}")
+    _check(r is None or (r.shape == x.shape and r.dtype == x.dtype), what, "x and the residual must share shape and dtype")
+    _check(len(copy_src) == len(copy_dst) <= 2, what, "at most two state copies")
+    x, weight = _prep(x), _prep(weight)
+    r = None if r is None else _prep(r)
+    y = torch.empty_like(x)
+    s = None if r is None else torch.empty_like(x)
+    copies = []
+    for a, b in zip(copy_src, copy_dst):
+        _check(a.dtype == b.dtype == torch.float32 and a.numel() == b.numel() and a.is_contiguous() and b.is_contiguous(),
+               what, "state copies are between contiguous float32 tensors of one size")
+        copies += [a.data_ptr(), b.data_ptr(), a.numel()]
+    copies += [None, None, 0] * (2 - len(copy_src))
+    rc = _lib.load().xl_add_rmsnorm_fwd(x.data_ptr(), _lib.ptr(r), weight.data_ptr(), _lib.ptr(s), y.data_ptr(),
+                                        x.numel() // max(D, 1), D, float(eps), *copies, _lib.dtype_code(x, what),
+                                        _lib.stream_of(x))
+    _lib.check(rc, what)
+    return s, y
+
+
+@torch.library.custom_op("xlstm_hip::rms_norm", mutates_args=())
+def rms_norm_op(x: Tensor, weight: Tensor, eps: float) -> Tensor:
+    """x / rms(x) * weight over the last axis, float32, rounded once (bf16 / f16)."""
+    return _add_rmsnorm(x, None, weight, eps, [], [], "rms_norm")[1]
+
+
+@rms_norm_op.register_fake
+def _(x, weight, eps):
+    return torch.empty_like(x, memory_format=torch.contiguous_format)
+
+
+@torch.library.custom_op("xlstm_hip::add_rmsnorm", mutates_args=("copy_dst",))
+def add_rmsnorm_op(x: Tensor, residual: Tensor, weight: Tensor, eps: float, copy_src: Sequence[Tensor],
+                   copy_dst: Sequence[Tensor]) -> tuple[Tensor, Tensor]:
+    """(x + residual, rms_norm of it); up to two float32 states copied along."""
+    return _add_rmsnorm(x, residual, weight, eps, copy_src, copy_dst, "add_rmsnorm")
+
+
+@add_rmsnorm_op.register_fake
+def _(x, residual, weight, eps, copy_src, copy_dst):
+    return tuple(torch.empty_like(x, memory_format=torch.contiguous_format) for _ in range(2))
+
+
+@torch.library.custom_op("xlstm_hip::silu_mul", mutates_args=())
+def silu_mul_op(gate: Tensor, up: Tensor) -> Tensor:
+    """silu(gate) * up, the SiLU rounded to the dtype first (bf16 / f16)."""
+    what = "silu_mul"
+    _lib.require_gpu(gate, up, what=what)
+    _check(gate.shape == up.shape and gate.dtype == up.dtype, what, "gate and up must share shape and dtype")
+    gate, up = _prep(gate), _prep(up)
+    y = torch.empty_like(gate)
+    rc = _lib.load().xl_silu_mul_fwd(gate.data_ptr(), up.data_ptr(), y.data_ptr(), y.numel(), _lib.dtype_code(y, what),
+                                     _lib.stream_of(y))
+    _lib.check(rc, what)
+    return y
+
+
+@silu_mul_op.register_fake
+def _(gate, up):
+    return torch.empty_like(gate, memory_format=torch.contiguous_format)
 
 
 # ------------------------------------------- logit projection + soft-cap epilogue

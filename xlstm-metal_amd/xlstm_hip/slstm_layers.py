@@ -10,7 +10,7 @@ reference root, ``SL`` = ``xlstm_metal/torch_native/blocks/slstm/slstm_layers``)
 * ``sLSTMProjectionCell`` (``SL/slstm_projection_cell.py:25-126``): the conv and
   its SiLU are one kernel on the channels-last input (no permuted copies); the
   gate projections with their soft-cap are ``gate_proj_kernel`` (i and f
-  stacked over the conv output, o over the input; float32 takes ``nn.Linear``
+  together over the conv output, o over the input; float32 takes ``nn.Linear``
   and ``soft_cap_kernel``); the z projection is ``nn.Linear`` (a library GEMM).
 * ``sLSTMOutputCell`` (``SL/slstm_output_cell.py:18-91``): the per-head
   ``nn.GroupNorm`` runs ``group_norm_kernel``; ``out_proj`` is ``nn.Linear``.
@@ -110,18 +110,16 @@ class sLSTMProjectionCell(nn.Module):
     def forward(self, x: Tensor) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
         """x [B, S, D] -> z [B, S, NH, H], i, f, o pre-activations [B, S, NH], x_conv [B, S, D].
 
-        i and f are one gate-projection kernel over x_conv (their weights stacked), o one over x."""
-        from .mlstm_layers import gate_proj_softcap, stacked_linears
+        i and f are one gate-projection kernel over x_conv, o one over x."""
+        from .mlstm_layers import gate_pair_softcap, gate_proj_softcap
         B, S, _ = x.shape
-        NH = self.num_heads
         x_conv = x if self.conv1d is None else self.conv1d.forward_channels_last(x, activation="silu")
         # the reference soft-caps with torch ops in x's dtype (slstm_projection_cell.py:84-89)
-        gif = gate_proj_softcap(x_conv, *stacked_linears(self.igate_proj, self.fgate_proj), self.gate_soft_cap,
-                                cap_in_dtype=True)
+        i, f = gate_pair_softcap(x_conv, self.igate_proj, self.fgate_proj, self.gate_soft_cap, cap_in_dtype=True)
         o_preact = gate_proj_softcap(x, self.ogate_proj.weight, self.ogate_proj.bias, self.gate_soft_cap,
                                      cap_in_dtype=True)
-        z = self.z_proj(x).view(B, S, NH, self.head_dim)
-        return z, gif[..., :NH], gif[..., NH:], o_preact, x_conv
+        z = self.z_proj(x).view(B, S, self.num_heads, self.head_dim)
+        return z, i, f, o_preact, x_conv
 
 
 class sLSTMOutputCell(nn.Module):

@@ -17,8 +17,8 @@ sigma(o), then out_proj).  The sLSTM layer is sLSTMProjectionCell (conv1d + SiLU
 kernels, z Linear) -> the sLSTM sequence kernel over the prompt and the step kernel per token
 -> sLSTMOutputCell (``group_norm_kernel``, out_proj).  The lm_head and the logit soft-cap are
 one kernel of this library (``lm_head_softcap``; ``fused_lm_head = False`` runs torch's Linear and
-then the soft_cap kernel instead).  Projections, FFN, norms and embedding are torch (hipBLASLt
-GEMMs); every mLSTM/sLSTM kernel is this library's.
+then the soft_cap kernel instead).  Projections, FFN and embedding are torch (hipBLASLt GEMMs), the
+blocks' norms with the residual before them and the SwiGLU product one pass each; every mLSTM/sLSTM kernel is this library's.
 
 Weights are N(0, init_std) in the model dtype (there is no checkpoint); the mLSTM forget-gate
 bias starts at +3 and the input-gate bias at 0, so the gates sit where a trained model keeps
@@ -32,7 +32,7 @@ Decoding keeps every state on the GPU and updates the mLSTM C state in place; on
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import List
+from typing import List, Optional
 
 import torch
 import torch.nn as nn
@@ -41,7 +41,8 @@ from torch import Tensor
 
 from .backend import (get_mlstm_kernel, get_mlstm_sequence_kernel, get_mlstm_step_kernel,
                       wrap_chunkwise__arbitrary_sequence_length)
-from .mlstm_layers import mLSTMOutputCell, mLSTMProjectionCell
+from .mlstm_layers import gate_pair_softcap, gate_proj_softcap, mLSTMOutputCell, mLSTMProjectionCell
+from .ops import add_rmsnorm_op, rms_norm_op, silu_mul_op
 from .recurrent import mlstm_recurrent_step_
 from .slstm import slstm_sequence, slstm_step
 from .slstm_layers import sLSTMOutputCell, sLSTMProjectionCell
@@ -98,6 +99,24 @@ CFG3_STACK = StackConfig("cfg3_xlstm7b", d_model=4096, num_blocks=32, mlstm_head
 CFG4_STACK = StackConfig("cfg4_mixed", d_model=2048, num_blocks=24, mlstm_heads=8, slstm_every=8)
 
 
+def _one_pass(x: Tensor, other: Tensor) -> bool:
+    """Whether the block's element-wise kernels (csrc/block_ops.hip) take x: GPU tensors of one 16-bit
+    dtype, rows of a multiple of 8 values, no gradient recorded (the kernels are forward-only)."""
+    return (x.device.type == "cuda" and x.dtype in (torch.bfloat16, torch.float16) and other.dtype == x.dtype
+            and x.shape[-1] % 8 == 0 and not (torch.is_grad_enabled() and (x.requires_grad or other.requires_grad)))
+
+
+def _add_norm(x: Tensor, r: Optional[Tensor], norm: "_RMSNorm", copies=()):
+    """(x + r, norm(x + r)), r None: (x, norm(x)); copies: up to two (source, destination) float32 states
+    copied by the same launch."""
+    if r is not None and _one_pass(x, norm.weight):
+        return add_rmsnorm_op(x, r, norm.weight, norm.eps, [s for s, _ in copies], [d for _, d in copies])
+    for s, d in copies:
+        d.copy_(s)
+    x = x if r is None else x + r
+    return x, norm(x)
+
+
 class _RMSNorm(nn.Module):
     """RMSNorm with the reduction in float32 (the reference's norm_reduce_force_float32 default)."""
 
@@ -107,6 +126,8 @@ class _RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: Tensor) -> Tensor:
+        if _one_pass(x, self.weight):
+            return rms_norm_op(x, self.weight, self.eps)
         return F.rms_norm(x.float(), (x.shape[-1],), self.weight.float(), self.eps).to(x.dtype)
 
 
@@ -118,7 +139,10 @@ class _FFN(nn.Module):
         self.proj_down = nn.Linear(hidden, d, bias=False)
 
     def forward(self, x: Tensor) -> Tensor:
-        return self.proj_down(F.silu(self.proj_up_gate(x)) * self.proj_up(x))
+        gate, up = self.proj_up_gate(x), self.proj_up(x)
+        if _one_pass(gate, up):
+            return self.proj_down(silu_mul_op(gate, up))
+        return self.proj_down(F.silu(gate) * up)
 
 
 @dataclass
@@ -156,19 +180,23 @@ class _mLSTMBlock(nn.Module):
         h, (C, n, m) = wrap_chunkwise__arbitrary_sequence_length(
             self._chunkwise, self._sequence, self._step, q.contiguous(), k.contiguous(), v.contiguous(),
             f.contiguous(), i.contiguous(), return_last_states=True, eps=self.cfg.eps)
-        x = x + self.out.out_proj(self.out.gated(h, xn))
-        return x + self.ffn(self.norm_ffn(x)), _MState(C.contiguous(), n.contiguous(), m.contiguous())
+        x, xn = _add_norm(x, self.out.out_proj(self.out.gated(h, xn)), self.norm_ffn)
+        return x + self.ffn(xn), _MState(C.contiguous(), n.contiguous(), m.contiguous())
 
     def decode(self, x: Tensor, st: _MState) -> Tensor:
         """x [B, 1, d]; updates st in place (C in place, n and m replaced)."""
-        xn = self.norm_mlstm(x)
+        return torch.add(*self.decode_split(x, st))
+
+    def decode_split(self, x: Tensor, st: _MState, r: Optional[Tensor] = None):
+        """decode() of x + r, returning the two terms of its result: the next norm adds them as it reads
+        them."""
+        x, xn = _add_norm(x, r, self.norm_mlstm)
         q, k, v, i, f = self.proj(xn)
         h, (_, n, m) = mlstm_recurrent_step_(q[:, :, 0], k[:, :, 0], v[:, :, 0], i, f, st.C, st.n, st.m,
                                              eps=self.cfg.eps)
-        st.n.copy_(n)
-        st.m.copy_(m)
-        x = x + self.out.out_proj(self.out.gated(h[:, :, None, :], xn))
-        return x + self.ffn(self.norm_ffn(x))
+        x, xn = _add_norm(x, self.out.out_proj(self.out.gated(h[:, :, None, :], xn)), self.norm_ffn,
+                          ((n, st.n), (m, st.m)))
+        return x, self.ffn(xn)
 
 
 class _sLSTMBlock(nn.Module):
@@ -191,31 +219,32 @@ class _sLSTMBlock(nn.Module):
         z, i, f, o, _ = self.proj(xn)
         h, (c, n, m) = slstm_sequence(z.contiguous(), i.contiguous(), f.contiguous(), o.contiguous(),
                                       eps=self.cfg.eps)
-        x = x + self.out(h)
+        x, xf = _add_norm(x, self.out(h), self.norm_ffn)
         conv = xn.new_zeros(B, K - 1, d)
         tail = xn[:, max(0, S - (K - 1)):]
         conv[:, K - 1 - tail.shape[1]:] = tail
-        return x + self.ffn(self.norm_ffn(x)), _SState(c.contiguous(), n.contiguous(), m.contiguous(), conv)
+        return x + self.ffn(xf), _SState(c.contiguous(), n.contiguous(), m.contiguous(), conv)
 
     def decode(self, x: Tensor, st: _SState) -> Tensor:
+        return torch.add(*self.decode_split(x, st))
+
+    def decode_split(self, x: Tensor, st: _SState, r: Optional[Tensor] = None):
         B = x.shape[0]
         NH, H = self.cfg.slstm_heads, self.H
-        xn = self.norm_slstm(x)
+        x, xn = _add_norm(x, r, self.norm_slstm)
         window = torch.cat([st.conv, xn], dim=1)          # [B, K, d]: the conv's receptive field
         p = self.proj
         x_conv = p.conv1d.forward_channels_last(window, activation="silu")[:, -1:]
-        from .mlstm_layers import gate_proj_softcap, stacked_linears
-        gif = gate_proj_softcap(x_conv, *stacked_linears(p.igate_proj, p.fgate_proj), p.gate_soft_cap,
-                                cap_in_dtype=True)
+        i, f = gate_pair_softcap(x_conv, p.igate_proj, p.fgate_proj, p.gate_soft_cap, cap_in_dtype=True)
         o = gate_proj_softcap(xn, p.ogate_proj.weight, p.ogate_proj.bias, p.gate_soft_cap, cap_in_dtype=True)
         z = p.z_proj(xn).view(B, NH, H)
-        h, c, n, m = slstm_step(z, gif[:, 0, :NH], gif[:, 0, NH:], o[:, 0], st.c, st.n, st.m, eps=self.cfg.eps)
+        h, c, n, m = slstm_step(z, i[:, 0], f[:, 0], o[:, 0], st.c, st.n, st.m, eps=self.cfg.eps)
         st.c.copy_(c)
         st.n.copy_(n)
         st.m.copy_(m)
         st.conv.copy_(window[:, 1:])
-        x = x + self.out(h.view(B, 1, NH, H))
-        return x + self.ffn(self.norm_ffn(x))
+        x, xn = _add_norm(x, self.out(h.view(B, 1, NH, H)), self.norm_ffn)
+        return x, self.ffn(xn)
 
 
 class xLSTMStack(nn.Module):
@@ -251,8 +280,8 @@ class xLSTMStack(nn.Module):
                     p.copy_(torch.randn(p.shape, generator=g, device=device) * cfg.init_std)
         return model.eval()
 
-    def logits(self, x: Tensor) -> Tensor:
-        xn = self.out_norm(x)
+    def logits(self, x: Tensor, r: Optional[Tensor] = None) -> Tensor:
+        _, xn = _add_norm(x, r, self.out_norm)
         if self.fused_lm_head:
             return lm_head_softcap(xn, self.lm_head.weight, self.cfg.logit_soft_cap)
         return soft_cap(self.lm_head(xn), self.cfg.logit_soft_cap)
@@ -270,10 +299,10 @@ class xLSTMStack(nn.Module):
     @torch.no_grad()
     def decode_step(self, token: Tensor, states: List) -> Tensor:
         """token [B] -> soft-capped logits [B, vocab]; states updated in place."""
-        x = self.embedding(token[:, None])
+        x, r = self.embedding(token[:, None]), None
         for blk, st in zip(self.blocks, states):
-            x = blk.decode(x, st)
-        return self.logits(x)[:, 0]
+            x, r = blk.decode_split(x, st, r)
+        return self.logits(x, r)[:, 0]
 
     @torch.no_grad()
     def generate(self, tokens: Tensor, steps: int, graph: bool = True) -> Tensor:
