@@ -141,6 +141,18 @@ int xl_mlstm_chunkwise_fwd(const void* q, const void* k, const void* v, const vo
                            void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The same with q, k, v read where a projection left them: strides = {batch, head, row} of q, of k, of v
+ * in elements (columns contiguous; multiples of 8; rows at least the head width apart).  Pipelined
+ * algorithm only (XL_ERR_UNSUPPORTED where xl_mlstm_chunkwise_algo names another).
+ */
+int xl_mlstm_chunkwise_fwd_strided(const void* q, const void* k, const void* v, const int64_t* strides,
+                                   const void* i, const void* f, const float* c0, const float* n0,
+                                   const float* m0, void* h, float* c_last, float* n_last, float* m_last,
+                                   int B, int NH, int S, int DQK, int DV, int L, float qk_scale, float eps,
+                                   int dtype_qkv, int dtype_gates, int algo,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Chunkwise mLSTM forward that allocates nothing and takes no workspace.  No
  * counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops or harnesses that

@@ -18,6 +18,7 @@ struct ChunkwiseArgs {
   void* stream;
   int max_segments;  // fused algorithm: at most this many sequence segments (1: no split)
   int pipelined;     // fused algorithm: the pipelined schedule (chunkwise_pipe.hip)
+  long long strides[9];  // pipelined schedule: batch, head and row strides of q, k, v in elements (rows 0: contiguous)
 };
 
 // Per-chunk gate prefix: sb[t] = sum_{u<=t} logsig(f_u) in sequential order

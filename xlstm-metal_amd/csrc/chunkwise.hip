@@ -92,6 +92,27 @@ extern "C" int xl_mlstm_chunkwise_algo(int B, int NH, int S, int DQK, int DV, in
   return chosen;
 }
 
+namespace xl {
+static int forward(ChunkwiseArgs& a, int algo) {
+  const int B = a.B, NH = a.NH, S = a.S, DQK = a.DQK, DV = a.DV, L = a.L;
+  int rc = chunkwise_check_args(a, algo);
+  if (rc) return rc;
+  int chosen = XL_CHUNKWISE_TWO_PASS;
+  rc = pick(a, algo, &chosen);
+  if (rc) return rc;
+  const bool fused = single_pass(chosen);
+  a.pipelined = chosen == XL_CHUNKWISE_PIPELINED;
+  const size_t need = fused ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments)
+                            : chunkwise_two_pass_workspace(B, NH, S, DQK, DV, L);
+  if (!a.workspace || a.workspace_bytes < need)
+    return set_error(XL_ERR_WORKSPACE, "xl_mlstm_chunkwise_fwd: %s workspace needs %zu bytes, got %zu",
+                     fused ? "fused" : "two-pass", need, a.workspace ? a.workspace_bytes : (size_t)0);
+  if (((uintptr_t)a.workspace) & 255u)
+    return set_error(XL_ERR_INVALID_ARG, "xl_mlstm_chunkwise_fwd: workspace must be 256-byte aligned");
+  return fused ? chunkwise_fused(a) : chunkwise_two_pass(a);
+}
+}  // namespace xl
+
 extern "C" int xl_mlstm_chunkwise_fwd(const void* q, const void* k, const void* v, const void* i, const void* f,
                                       const float* c0, const float* n0, const float* m0, void* h, float* c_last,
                                       float* n_last, float* m_last, int B, int NH, int S, int DQK, int DV, int L,
@@ -102,19 +123,36 @@ extern "C" int xl_mlstm_chunkwise_fwd(const void* q, const void* k, const void* 
   ChunkwiseArgs a = {q, k, v, i, f, c0, n0, m0, h, c_last, n_last, m_last, B, NH, S, DQK, DV, L,
                      qk_scale, eps, dtype_qkv, dtype_gates, workspace, workspace_bytes, stream,
                      kChunkwiseMaxSegments};
+  return forward(a, algo);
+}
+
+extern "C" int xl_mlstm_chunkwise_fwd_strided(const void* q, const void* k, const void* v, const int64_t* strides,
+                                              const void* i, const void* f, const float* c0, const float* n0,
+                                              const float* m0, void* h, float* c_last, float* n_last, float* m_last,
+                                              int B, int NH, int S, int DQK, int DV, int L, float qk_scale, float eps,
+                                              int dtype_qkv, int dtype_gates, int algo, void* workspace,
+                                              size_t workspace_bytes, void* stream) {
+  using namespace xl;
+  clear_error();
+  const char* who = "xl_mlstm_chunkwise_fwd_strided";
+  ChunkwiseArgs a = {q, k, v, i, f, c0, n0, m0, h, c_last, n_last, m_last, B, NH, S, DQK, DV, L,
+                     qk_scale, eps, dtype_qkv, dtype_gates, workspace, workspace_bytes, stream,
+                     kChunkwiseMaxSegments};
+  if (!strides) return set_error(XL_ERR_INVALID_ARG, "%s: null strides", who);
+  for (int t = 0; t < 3; ++t) {
+    const int64_t *s = strides + 3 * t, width = t < 2 ? DQK : DV;
+    // rows must not overlap (a row past a ragged end then lies past the records) and a chunk's byte
+    // offsets stay in 31 bits
+    if (s[0] < 0 || s[1] < 0 || s[2] < width || s[2] > (1 << 22) || ((s[0] | s[1] | s[2]) & 7))
+      return set_error(XL_ERR_INVALID_ARG, "%s: strides must be multiples of 8 elements, rows at least the width and at most 2^22 apart", who);
+    for (int d = 0; d < 3; ++d) a.strides[3 * t + d] = s[d];
+  }
   int rc = chunkwise_check_args(a, algo);
   if (rc) return rc;
   int chosen = XL_CHUNKWISE_TWO_PASS;
   rc = pick(a, algo, &chosen);
   if (rc) return rc;
-  const bool fused = single_pass(chosen);
-  a.pipelined = chosen == XL_CHUNKWISE_PIPELINED;
-  const size_t need = fused ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments)
-                            : chunkwise_two_pass_workspace(B, NH, S, DQK, DV, L);
-  if (!workspace || workspace_bytes < need)
-    return set_error(XL_ERR_WORKSPACE, "xl_mlstm_chunkwise_fwd: %s workspace needs %zu bytes, got %zu",
-                     fused ? "fused" : "two-pass", need, workspace ? workspace_bytes : (size_t)0);
-  if (((uintptr_t)workspace) & 255u)
-    return set_error(XL_ERR_INVALID_ARG, "xl_mlstm_chunkwise_fwd: workspace must be 256-byte aligned");
-  return fused ? chunkwise_fused(a) : chunkwise_two_pass(a);
+  if (chosen != XL_CHUNKWISE_PIPELINED)
+    return set_error(XL_ERR_UNSUPPORTED, "%s: only the pipelined algorithm reads strided q, k, v", who);
+  return forward(a, XL_CHUNKWISE_PIPELINED);
 }

@@ -754,6 +754,9 @@ static int launch(const ChunkwiseArgs& A) {
     return XL_OK;
   };
   const bf16_t *q = (const bf16_t*)A.q, *k = (const bf16_t*)A.k, *v = (const bf16_t*)A.v;
+  const int strided = A.strides[2] != 0;
+  auto strides = [&](int i) { return Strides{A.strides[3 * i], A.strides[3 * i + 1], (int)A.strides[3 * i + 2]}; };
+  const Strides qs = strides(0), ks = strides(1), vs = strides(2);
   SegArgs sg = {1, NC, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   if (lay.P > 1) {
     // pass 1: every segment but the last, states only (segment 0 from the caller's initial
@@ -768,7 +771,7 @@ static int launch(const ChunkwiseArgs& A) {
     float* sms = sns + (lay.P - 1) * nst;
     SegArgs s1 = {lay.P - 1, lay.kc_per_seg, nullptr, nullptr, nullptr, ec, en, em};
     const MainArgs m1 = {q, k, v, A.c0, A.n0, A.m0, nullptr, nullptr, nullptr, nullptr, prep,
-                         A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, s1, A.DQK};
+                         A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, s1, A.DQK, A.NH, strided, qs, ks, vs};
     const int rc = main(true, (unsigned)(BNH * nvtile * (lay.P - 1)), m1);
     if (rc) return rc;
     const int per4 = (A.DQK * A.DV + A.DQK) / 4;
@@ -777,7 +780,7 @@ static int launch(const ChunkwiseArgs& A) {
     sg = SegArgs{lay.P, lay.kc_per_seg, scs, sns, sms, nullptr, nullptr, nullptr};
   }
   const MainArgs m2 = {q, k, v, A.c0, A.n0, A.m0, (bf16_t*)A.h, A.c_last, A.n_last, A.m_last, prep,
-                       A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, sg, A.DQK};
+                       A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, sg, A.DQK, A.NH, strided, qs, ks, vs};
   const int rc = main(false, (unsigned)(BNH * nvtile * sg.nseg), m2);
   if (rc) return rc;
   return check_launch(A.pipelined ? "xl_mlstm_chunkwise_fwd(pipelined)" : "xl_mlstm_chunkwise_fwd(fused)");

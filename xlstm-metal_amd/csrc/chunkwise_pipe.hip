@@ -108,7 +108,10 @@ __device__ __forceinline__ int state_row(int dw0, int dt, int l32) {
   return dw0 + 32 * dt + 16 * (l32 >> 4) + 8 * ((x >> 2) & 1) + 4 * (x >> 3) + (x & 3);
 }
 
-template <typename T, int DQK, bool STATES_ONLY>
+// STRIDED: q, k, v rows at a.qs / ks / vs (a projection's views, read in place); otherwise contiguous
+// [B, NH, S, D], a case of its own because the pitches and record lengths of the strided form cost the
+// main loop's scalar registers 1.3 % (454 -> 460 us at B4 NH8 S8192 DQK256 DV512).
+template <typename T, int DQK, bool STATES_ONLY, bool STRIDED>
 __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a) {
   using SM = Smem<DQK>;
   using E = Elt<T>;
@@ -151,15 +154,20 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
   bf16_t* nbuf = (bf16_t*)(smem + SM::NB);   // [2][4][NB_PITCH]: n parts entering chunk kc live in buffer kc & 1
   float* gbuf = (float*)(smem + SM::GATES);  // [2][GROWS][64]: rows of chunk kc live in buffer kc & 1
 
-  const bf16_t* qh = a.q + (size_t)bh * S * dq;
-  const bf16_t* kh = a.k + (size_t)bh * S * dq;
-  const bf16_t* vh = a.v + (size_t)bh * S * DV;
+  const int b = STRIDED ? bh / a.NH : 0, hd = STRIDED ? bh - b * a.NH : 0;
+  const bf16_t* qh = a.q + (STRIDED ? b * a.qs.batch + hd * a.qs.head : (long long)bh * S * dq);
+  const bf16_t* kh = a.k + (STRIDED ? b * a.ks.batch + hd * a.ks.head : (long long)bh * S * dq);
+  const bf16_t* vh = a.v + (STRIDED ? b * a.vs.batch + hd * a.vs.head : (long long)bh * S * DV);
+  const int qp = STRIDED ? a.qs.row : dq, kp = STRIDED ? a.ks.row : dq, vp = STRIDED ? a.vs.row : DV;  // row pitches
+  auto rows_rsrc = [](const bf16_t* base, int rows, int pitch, int width) {
+    return STRIDED ? chunk_rsrc_strided(base, rows, pitch * 2, width * 2) : chunk_rsrc(base, rows, pitch * 2);
+  };
   bf16_t* hh = a.h + (size_t)bh * S * DV;
   // valid rows of chunk kc (0 past the sequence: a chunk past the end gets a buffer resource
   // with no records, so its prefetches return zeros without touching memory; they are issued
   // unconditionally, which keeps the compiler's load counters exact)
   auto rows_of = [&](int kc) { return __builtin_amdgcn_readfirstlane(max(0, min(L, S - kc * L))); };
-  auto q_rsrc = [&](int kc) { return chunk_rsrc(qh + (size_t)kc * L * dq, rows_of(kc), dq * 2); };
+  auto q_rsrc = [&](int kc) { return rows_rsrc(qh + (size_t)kc * L * qp, rows_of(kc), qp, dq); };
 
   if (w < NSW) {
     // =====================================================================
@@ -228,14 +236,14 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
     // q fragments (B operand of the transposed product C^T Q^T): token 32 tt + l32,
     // rows dw0 + 16 s + 8 hh .. +7
     u32x4 Qs[2][QKS];
-    const uint32_t qs_off = (uint32_t)((l32 * dq + dw0 + 8 * hh) * 2);
+    const uint32_t qs_off = (uint32_t)((l32 * qp + dw0 + 8 * hh) * 2);
     auto load_qs = [&](int kc) {
       const auto rq = q_rsrc(kc);
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int s = 0; s < QKS; ++s)
-          Qs[tt][s] = ld16s(rq, qs_off, (uint32_t)((32 * tt * dq + 16 * s) * 2));
+          Qs[tt][s] = ld16s(rq, qs_off, (uint32_t)((32 * tt * qp + 16 * s) * 2));
     };
     if (!STATES_ONLY) load_qs(kc0);
     __syncthreads();  // B0: tiles, gate rows and n parts of the first chunk
@@ -457,16 +465,16 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
     // piece u * NOT + t: K row (piece / (DQK / 8)), 16-byte column piece % (DQK / 8) of the
     // tile (NOT / (DQK / 8) rows further per u); in memory rows of dq, so a column past dq
     // gets an offset beyond the buffer's records and reads as zero; V row piece >> 3, 8 columns
-    const uint32_t k_off = (t % (DQK / 8)) < dq / 8 ? (uint32_t)((t / (DQK / 8)) * dq * 2 + 16 * (t % (DQK / 8)))
+    const uint32_t k_off = (t % (DQK / 8)) < dq / 8 ? (uint32_t)((t / (DQK / 8)) * kp * 2 + 16 * (t % (DQK / 8)))
                                                      : 0x80000000u;
-    const uint32_t v_off = (uint32_t)(((t >> 3) * DV + v0 + 8 * (t & 7)) * 2);
+    const uint32_t v_off = (uint32_t)(((t >> 3) * vp + v0 + 8 * (t & 7)) * 2);
     auto load_kv = [&](int kc) {
-      const auto r = chunk_rsrc(kh + (size_t)kc * L * dq, rows_of(kc), dq * 2);
+      const auto r = rows_rsrc(kh + (size_t)kc * L * kp, rows_of(kc), kp, dq);
 #pragma unroll
-      for (int u = 0; u < NKO; ++u) Kst[u] = ld16s(r, k_off, (uint32_t)(u * (NOT / (DQK / 8)) * dq * 2));
-      const auto rv = chunk_rsrc(vh + (size_t)kc * L * DV, rows_of(kc), DV * 2);
+      for (int u = 0; u < NKO; ++u) Kst[u] = ld16s(r, k_off, (uint32_t)(u * (NOT / (DQK / 8)) * kp * 2));
+      const auto rv = rows_rsrc(vh + (size_t)kc * L * vp, rows_of(kc), vp, DV);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) Vst[u] = ld16s(rv, v_off, (uint32_t)(u * (NOT / 8) * DV * 2));  // NOT / 8 rows per u
+      for (int u = 0; u < 2; ++u) Vst[u] = ld16s(rv, v_off, (uint32_t)(u * (NOT / 8) * vp * 2));  // NOT / 8 rows per u
     };
     auto store_kv = [&]() {
 #pragma unroll
@@ -511,7 +519,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
     auto out_wave = [&](auto otag) {
       constexpr int o = decltype(otag)::value;
       u32x4 Qf[KPD];
-      const uint32_t qf_off = (uint32_t)(((16 * o + r16) * dq + 8 * g) * 2);
+      const uint32_t qf_off = (uint32_t)(((16 * o + r16) * qp + 8 * g) * 2);
       float pv[5];  // gate prep of the next chunk
       // q fragments of rows 16o + r16 for S: k-slice 32p + 8g .. 32p + 8g + 7 (one
       // 16-byte load; the K operand below uses the same contiguous k order)
@@ -665,7 +673,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
 template <typename T, int DQK, bool STATES_ONLY>
 static int launch_one(unsigned nwg, hipStream_t st, const MainArgs& a) {
   const size_t smem = Smem<DQK>::BYTES;
-  auto kern = chunkwise_pipe_kernel<T, DQK, STATES_ONLY>;
+  auto kern = a.strided ? chunkwise_pipe_kernel<T, DQK, STATES_ONLY, true> : chunkwise_pipe_kernel<T, DQK, STATES_ONLY, false>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess)
     return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_fwd: LDS attribute failed: %s", hipGetErrorString(e));

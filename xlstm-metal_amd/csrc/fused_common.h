@@ -79,6 +79,12 @@ __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc(const bf16_t* base, int rows, int row_bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), (short)0, rows * row_bytes, 0x00020000);
 }
+// The same for rows `pitch` bytes apart of which `width` bytes belong to the tensor (a [B, S, NH, D]
+// projection read in place): the records end with the last valid row, so rows past it read as zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t chunk_rsrc_strided(const bf16_t* base, int rows, int pitch, int width) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), (short)0, rows > 0 ? (rows - 1) * pitch + width : 0,
+                                           0x00020000);
+}
 __device__ __forceinline__ u32x4 ld16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
@@ -165,6 +171,12 @@ struct Smem {
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
 
+// Where row t of head h of batch b starts: b * batch + h * head + t * row elements (columns contiguous).
+struct Strides {
+  long long batch, head;
+  int row;
+};
+
 // Everything the main chunkwise kernels take (one (head, column tile, segment) per workgroup).
 struct MainArgs {
   const bf16_t *q, *k, *v;
@@ -176,6 +188,9 @@ struct MainArgs {
   float qk_scale, eps;
   SegArgs sg;
   int dq;  // q / k width in memory (DQK of the launch, or less: a multiple of DQK / 4)
+  int NH;
+  int strided;         // pipelined kernel: q, k, v at these strides (elements), else contiguous
+  Strides qs, ks, vs;
 };
 
 // The pipelined main kernel (chunkwise_pipe.hip): nwg workgroups of NTHREADS on stream st.

@@ -33,6 +33,8 @@ SIGNATURES = {
     "xl_mlstm_chunkwise_algo": (_i, [_i] * 8),
     "xl_mlstm_chunkwise_fwd": (_i, [_vp] * 5 + [_fp] * 3 + [_vp] + [_fp] * 3 + [_i] * 6 + [_f, _f] + [_i] * 3
                                + [_vp, _sz, _vp]),
+    "xl_mlstm_chunkwise_fwd_strided": (_i, [_vp] * 3 + [ctypes.POINTER(_i64)] + [_vp] * 2 + [_fp] * 3 + [_vp] + [_fp] * 3
+                                       + [_i] * 6 + [_f, _f] + [_i] * 3 + [_vp, _sz, _vp]),
     "xl_mlstm_chunkwise_bwd_workspace_size": (_sz, [_i] * 6),
     "xl_mlstm_chunkwise_bwd": (_i, [_vp] * 5 + [_fp] * 3 + [_vp, _fp] + [_vp] * 5 + [_fp] + [_i] * 6 + [_f, _f]
                                + [_i, _i, _vp, _sz, _vp]),

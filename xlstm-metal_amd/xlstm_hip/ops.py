@@ -9,6 +9,7 @@ no CPU path: CPU tensors raise.
 
 from __future__ import annotations
 
+import ctypes
 import warnings
 from typing import List, Optional, Sequence
 
@@ -190,6 +191,18 @@ def chunkwise_workspace_bytes(B, NH, S, DQK, DV, L, dtype, algo="auto") -> int:
                                                              _lib.ALGO[algo]))
 
 
+def _row_strides(*tensors):
+    """{batch, head, row} strides of each [B, NH, S, D] tensor for the pipelined kernel, None where one of
+    them has to be copied: columns contiguous, 16-byte rows and base, rows apart."""
+    out = []
+    for t in tensors:
+        s = [st if n > 1 else 0 for st, n in zip(t.stride()[:2], t.shape)] + [t.stride(2)]  # unused strides: 0
+        if t.stride(3) != 1 or (s[0] | s[1] | s[2]) & 7 or not t.shape[3] <= s[2] <= 1 << 22 or t.data_ptr() & 15:
+            return None
+        out += s
+    return (ctypes.c_int64 * 9)(*out)
+
+
 def _state_outs(ret, B, NH, DQK, DV, dev):
     if not ret:  # three distinct empties: custom-op outputs may not alias each other
         return tuple(torch.empty(_EMPTY_SHAPE, dtype=torch.float32, device=dev) for _ in range(3))
@@ -207,18 +220,28 @@ def mlstm_chunkwise_op(q: Tensor, k: Tensor, v: Tensor, i: Tensor, f: Tensor, c0
     B, NH, S, DQK, DV = _seq_shapes(q, k, v, i, f, c0, n0, m0, what)
     if S % chunk_size != 0 and algo not in (_lib.ALGO["fused"], _lib.ALGO["pipelined"]):  # single pass: ragged last chunk OK
         raise AssertionError(f"Sequence length {S} is not divisible by chunk size {chunk_size}.")
-    q, k, v, i, f = (_prep(t) for t in (q, k, v, i, f))
+    lib = _lib.load()
+    dq = _lib.dtype_code(q, what)
+    # q, k, v as a projection's permuted views: the pipelined kernel reads them in place
+    strides = None
+    if q.dtype != torch.float32 and not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
+        strides = _row_strides(q, k, v)
+        if strides is not None and int(lib.xl_mlstm_chunkwise_algo(B, NH, S, DQK, DV, chunk_size, dq,
+                                                                   int(algo))) != _lib.ALGO["pipelined"]:
+            strides = None
+    if strides is None:
+        q, k, v = (_prep(t) for t in (q, k, v))
+    i, f = _prep(i), _prep(f)
     c0, n0, m0 = _f32(c0), _f32(n0), _f32(m0)
     h = torch.empty((B, NH, S, DV), dtype=q.dtype, device=q.device)
     cl, nl, ml = _state_outs(return_last_states, B, NH, DQK, DV, q.device)
-    lib = _lib.load()
-    dq = _lib.dtype_code(q, what)
     if algo == _lib.ALGO["auto"] and q.dtype != torch.float32:
         _warn_slow_fallback(B, NH, S, DQK, DV, chunk_size, q.dtype)
     ws_bytes = int(lib.xl_mlstm_chunkwise_workspace_size(B, NH, S, DQK, DV, chunk_size, dq, int(algo)))
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None
-    rc = lib.xl_mlstm_chunkwise_fwd(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), i.data_ptr(), f.data_ptr(),
+    fwd = lib.xl_mlstm_chunkwise_fwd if strides is None else lib.xl_mlstm_chunkwise_fwd_strided
+    rc = fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), *(() if strides is None else (strides,)), i.data_ptr(), f.data_ptr(),
         _lib.ptr(c0), _lib.ptr(n0), _lib.ptr(m0), h.data_ptr(),
         cl.data_ptr() if return_last_states else None, nl.data_ptr() if return_last_states else None,
         ml.data_ptr() if return_last_states else None,

@@ -178,8 +178,7 @@ class _mLSTMBlock(nn.Module):
         xn = self.norm_mlstm(x)
         q, k, v, i, f = self.proj(xn)
         h, (C, n, m) = wrap_chunkwise__arbitrary_sequence_length(
-            self._chunkwise, self._sequence, self._step, q.contiguous(), k.contiguous(), v.contiguous(),
-            f.contiguous(), i.contiguous(), return_last_states=True, eps=self.cfg.eps)
+            self._chunkwise, self._sequence, self._step, q, k, v, f, i, return_last_states=True, eps=self.cfg.eps)
         x, xn = _add_norm(x, self.out.out_proj(self.out.gated(h, xn)), self.norm_ffn)
         return x + self.ffn(xn), _MState(C.contiguous(), n.contiguous(), m.contiguous())
 
