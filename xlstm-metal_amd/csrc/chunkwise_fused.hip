@@ -701,6 +701,37 @@ static int segments_for(int B, int NH, int S, int DV, int max_seg) {
   return P < 2 ? 1 : P;
 }
 
+// The pipelined kernel's split (SplitArgs): w = 0 where one launch over the whole sequence is expected
+// to be no slower.  Costs in chunk times of a complete segment: a states-only chunk takes 0.55 of one
+// (B1 NH8 DQK256 DV512: 1.95 of 3.45 us; 1.5 of 2.9 at DQK128 DV256), a launch 1.5 beside its chunks (first loads,
+// last stores), an end state read at a start 0.3.  Segment 0 (complete) and the states-only segments share
+// a launch, so n0 = 0.55 n fills both; the chunks left over make n0 longer or the last segment shorter.
+// Measured against equal segments behind a states-only pass over all but the last and a combine launch:
+// B1 NH8 S2011 DQK256 DV512 65.4 -> 51.9 us a call (57.8 of them without the zero fills of the initial state),
+// the forward of B2 NH8 S4096 186 -> 158 us.
+struct Split {
+  int w, n0, n;
+};
+static Split pipe_split(int B, int NH, int S, int DV, int max_seg) {
+  const long long pairs = (long long)B * NH * (DV / DVT);
+  const int NC = (S + L - 1) / L;
+  Split best = {0, NC, 0};
+  if (pairs <= 0 || pairs * 2 > kTargetWorkgroups || max_seg < 2) return best;
+  constexpr float STATE = 0.55f, LAUNCH = 1.5f, START = 0.3f;
+  float cost = 0.9f * (LAUNCH + NC);  // a split has to be worth its second launch
+  const int wmax = min((int)(kTargetWorkgroups / pairs), min(kMaxSegments, max_seg) - 1);
+  for (int w = 2; w <= wmax; ++w) {
+    const int near = (int)(NC / (w + STATE));
+    for (int n = max(near, 1); n <= near + 1; ++n) {
+      const int n0 = max(NC - w * n, 1);
+      if (n0 + (w - 1) * n >= NC) continue;  // an empty last segment
+      const float c = 2 * LAUNCH + START * w + fmaxf((float)n0, STATE * n) + n;
+      if (c < cost) cost = c, best = {w, n0, n};
+    }
+  }
+  return best;
+}
+
 struct Layout {  // workspace: gate prep, then (split only) the end states and start states
   int P, kc_per_seg;
   size_t prep_bytes, states_bytes, total;
@@ -721,6 +752,34 @@ static Layout layout_for(int B, int NH, int S, int DQK, int DV, int max_seg) {
   return l;
 }
 
+// bytes of the pipelined kernel's end states (C, n, m, total log forget gate per segment and head)
+static size_t split_bytes(int B, int NH, int S, int DQK, int DV, int max_seg) {
+  const Split sp = pipe_split(B, NH, S, DV, max_seg);
+  return align256((size_t)sp.w * B * NH * ((size_t)DQK * DV + DQK + 2) * sizeof(float));
+}
+
+static int launch_pipe(const ChunkwiseArgs& A, int DQK, float* prep) {
+  const int BNH = A.B * A.NH, NC = (A.S + L - 1) / L;
+  const Split s = pipe_split(A.B, A.NH, A.S, A.DV, A.max_segments);
+  const int strided = A.strides[2] != 0;
+  auto strides = [&](int i) { return Strides{A.strides[3 * i], A.strides[3 * i + 1], (int)A.strides[3 * i + 2]}; };
+  SplitArgs sp = {max(s.w, 1), s.n0, s.n, nullptr, nullptr, nullptr, nullptr};
+  if (s.w) {
+    sp.ec = (float*)((char*)A.workspace + layout_for(A.B, A.NH, A.S, A.DQK, A.DV, A.max_segments).prep_bytes);
+    sp.en = sp.ec + (size_t)s.w * BNH * A.DQK * A.DV;
+    sp.em = sp.en + (size_t)s.w * BNH * A.DQK;
+    sp.eg = sp.em + (size_t)s.w * BNH;
+  }
+  const MainArgs m = {(const bf16_t*)A.q, (const bf16_t*)A.k, (const bf16_t*)A.v, A.c0, A.n0, A.m0, (bf16_t*)A.h, A.c_last,
+                      A.n_last, A.m_last, prep, A.S, NC, A.DV, BNH, A.DV / DVT, A.qk_scale, A.eps, {}, A.DQK, A.NH, strided,
+                      strides(0), strides(1), strides(2), sp};
+  const bool f16 = A.dtype_qkv == XL_DTYPE_F16;
+  hipStream_t st = (hipStream_t)A.stream;
+  int rc = pipe_launch(f16, DQK, s.w ? PIPE_FIRST : PIPE_FULL, st, m);
+  if (!rc && s.w) rc = pipe_launch(f16, DQK, PIPE_LAST, st, m);
+  return rc ? rc : check_launch("xl_mlstm_chunkwise_fwd(pipelined)");
+}
+
 template <typename TG, int DQK>
 static int launch(const ChunkwiseArgs& A) {
   const int BNH = A.B * A.NH;
@@ -732,17 +791,16 @@ static int launch(const ChunkwiseArgs& A) {
   const int total = BNH * NC;
   hipLaunchKernelGGL(gate_prep_kernel<TG>, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, (const TG*)A.i,
                      (const TG*)A.f, prep, total, NC, A.S);
+  if (A.pipelined) return launch_pipe(A, DQK, prep);
   const size_t smem = Smem<DQK>::BYTES;
-  if (!A.pipelined) {
+  {
     for (auto kern : {chunkwise_fused_kernel<DQK, false>, chunkwise_fused_kernel<DQK, true>}) {
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
       if (e != hipSuccess)
         return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_fwd: LDS attribute failed: %s", hipGetErrorString(e));
     }
   }
-  // the main kernel: the pipelined schedule (chunkwise_pipe.hip) or the fused one
   auto main = [&](bool states_only, unsigned nwg, const MainArgs& m) -> int {
-    if (A.pipelined) return pipe_launch(A.dtype_qkv == XL_DTYPE_F16, DQK, states_only, nwg, st, m);
     if (states_only)
       hipLaunchKernelGGL((chunkwise_fused_kernel<DQK, true>), dim3(nwg), dim3(NTHREADS), smem, st, m.q, m.k, m.v,
                          m.c0, m.n0, m.m0, m.h, m.c_last, m.n_last, m.m_last, m.prep, m.S, m.NC, m.DV, m.BNH,
@@ -754,9 +812,6 @@ static int launch(const ChunkwiseArgs& A) {
     return XL_OK;
   };
   const bf16_t *q = (const bf16_t*)A.q, *k = (const bf16_t*)A.k, *v = (const bf16_t*)A.v;
-  const int strided = A.strides[2] != 0;
-  auto strides = [&](int i) { return Strides{A.strides[3 * i], A.strides[3 * i + 1], (int)A.strides[3 * i + 2]}; };
-  const Strides qs = strides(0), ks = strides(1), vs = strides(2);
   SegArgs sg = {1, NC, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   if (lay.P > 1) {
     // pass 1: every segment but the last, states only (segment 0 from the caller's initial
@@ -771,7 +826,7 @@ static int launch(const ChunkwiseArgs& A) {
     float* sms = sns + (lay.P - 1) * nst;
     SegArgs s1 = {lay.P - 1, lay.kc_per_seg, nullptr, nullptr, nullptr, ec, en, em};
     const MainArgs m1 = {q, k, v, A.c0, A.n0, A.m0, nullptr, nullptr, nullptr, nullptr, prep,
-                         A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, s1, A.DQK, A.NH, strided, qs, ks, vs};
+                         A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, s1, A.DQK, A.NH, 0, {}, {}, {}, {}};
     const int rc = main(true, (unsigned)(BNH * nvtile * (lay.P - 1)), m1);
     if (rc) return rc;
     const int per4 = (A.DQK * A.DV + A.DQK) / 4;
@@ -780,10 +835,10 @@ static int launch(const ChunkwiseArgs& A) {
     sg = SegArgs{lay.P, lay.kc_per_seg, scs, sns, sms, nullptr, nullptr, nullptr};
   }
   const MainArgs m2 = {q, k, v, A.c0, A.n0, A.m0, (bf16_t*)A.h, A.c_last, A.n_last, A.m_last, prep,
-                       A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, sg, A.DQK, A.NH, strided, qs, ks, vs};
+                       A.S, NC, A.DV, BNH, nvtile, A.qk_scale, A.eps, sg, A.DQK, A.NH, 0, {}, {}, {}, {}};
   const int rc = main(false, (unsigned)(BNH * nvtile * sg.nseg), m2);
   if (rc) return rc;
-  return check_launch(A.pipelined ? "xl_mlstm_chunkwise_fwd(pipelined)" : "xl_mlstm_chunkwise_fwd(fused)");
+  return check_launch("xl_mlstm_chunkwise_fwd(fused)");
 }
 
 template <typename TG>
@@ -794,7 +849,8 @@ static int launch_d(const ChunkwiseArgs& A) {  // the tile: 128 rows for DQK <= 
 }  // namespace fused
 
 size_t chunkwise_fused_workspace(int B, int NH, int S, int DQK, int DV, int max_segments) {
-  return fused::layout_for(B, NH, S, DQK, DV, max_segments).total;
+  const fused::Layout l = fused::layout_for(B, NH, S, DQK, DV, max_segments);
+  return max(l.total, l.prep_bytes + fused::split_bytes(B, NH, S, DQK, DV, max_segments));
 }
 
 int chunkwise_fused_segments(int B, int NH, int S, int DQK, int DV, int max_segments) {

@@ -111,7 +111,7 @@ __device__ __forceinline__ int state_row(int dw0, int dt, int l32) {
 // STRIDED: q, k, v rows at a.qs / ks / vs (a projection's views, read in place); otherwise contiguous
 // [B, NH, S, D], a case of its own because the pitches and record lengths of the strided form cost the
 // main loop's scalar registers 1.3 % (454 -> 460 us at B4 NH8 S8192 DQK256 DV512).
-template <typename T, int DQK, bool STATES_ONLY, bool STRIDED>
+template <typename T, int DQK, int MODE, bool STRIDED>
 __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a) {
   using SM = Smem<DQK>;
   using E = Elt<T>;
@@ -125,27 +125,38 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
   const int w = tid >> 6, lane = tid & 63;
   const int r16 = lane & 15, g = lane >> 4;
   const int ws = w & 3;  // index within the state or output group
-  const SegArgs& sg = a.sg;
+  const SplitArgs& sp = a.sp;
   const int S = a.S, NC = a.NC, DV = a.DV, BNH = a.BNH, nvtile = a.nvtile;
   // the head's q / k width in memory: DQK, or less (a multiple of DW) with the tile's rows and
   // columns past it zero (state waves past it idle, q and k read as zero there)
   const int dq = a.dq;
 
   // ---- XCD-aware workgroup -> (head, column tile): consecutive tiles of a head share an XCD
-  const int nwg = BNH * nvtile * sg.nseg;
+  const int nwg = BNH * nvtile * sp.w;
   int lin = blockIdx.x;
   if ((nwg & 7) == 0) lin = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);
-  const int bhs = lin / nvtile;  // segment * BNH + head
-  const int v0 = (lin - bhs * nvtile) * DVT;
-  const int seg = bhs / BNH, bh = bhs - seg * BNH;
-  const int kc0 = seg * sg.kc_per_seg, kc1 = min(NC, kc0 + sg.kc_per_seg);  // this segment's chunks
+  // (and a head's segments, whose start states read the same end states)
+  const int per_head = nvtile * sp.w;
+  const int bh = lin / per_head, in_head = lin - bh * per_head;
+  const int seg0 = in_head / nvtile, seg = seg0 + (MODE == PIPE_LAST ? 1 : 0);
+  const int v0 = (in_head - seg0 * nvtile) * DVT;
+  // this segment's chunks (PIPE_FULL: w = 1, n0 = NC; its bounds left to run time: with constants the
+  // compiler's order of the main loop runs 0.5 % slower), and whether only its end state is wanted
+  const int kc0 = seg == 0 ? 0 : sp.n0 + (seg - 1) * sp.n;
+  const int kc1 = seg == 0 ? sp.n0 : min(NC, kc0 + sp.n);
+  const bool states_only = MODE == PIPE_FIRST && seg != 0;
   const size_t cst = (size_t)BNH * dq * DV, nst = (size_t)BNH * dq;
-  const float* ci = seg == 0 ? a.c0 : (sg.sc ? sg.sc + (seg - 1) * cst : nullptr);
-  const float* ni = seg == 0 ? a.n0 : (sg.sn ? sg.sn + (seg - 1) * nst : nullptr);
-  const float m_init = seg == 0 ? (a.m0 ? a.m0[bh] : 0.f) : (sg.sm ? sg.sm[(seg - 1) * BNH + bh] : -INFINITY);
-  float* ce = sg.ec ? sg.ec + seg * cst : (seg == sg.nseg - 1 ? a.c_last : nullptr);
-  float* ne = sg.ec ? sg.en + seg * nst : a.n_last;
-  float* me = sg.ec ? sg.em + (size_t)seg * BNH : a.m_last;
+  float m_init = MODE != PIPE_LAST && seg == 0 ? (a.m0 ? a.m0[bh] : 0.f) : -INFINITY;
+  if (MODE == PIPE_LAST) {  // max over the end states before this segment
+    float G = 0.f;
+    for (int s = seg - 1; s >= 0; --s) {
+      m_init = fmaxf(m_init, sp.em[(size_t)s * BNH + bh] + G);
+      G += sp.eg[(size_t)s * BNH + bh];
+    }
+  }
+  float* ce = MODE == PIPE_FIRST ? sp.ec + seg * cst : seg0 == sp.w - 1 ? a.c_last : nullptr;
+  float* ne = MODE == PIPE_FIRST ? sp.en + seg * nst : a.n_last;
+  float* me = MODE == PIPE_FIRST ? sp.em + (size_t)seg * BNH : a.m_last;
 
   char* kn = smem + SM::KN;
   char* vn = smem + SM::VN;
@@ -169,6 +180,49 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
   auto rows_of = [&](int kc) { return __builtin_amdgcn_readfirstlane(max(0, min(L, S - kc * L))); };
   auto q_rsrc = [&](int kc) { return rows_rsrc(qh + (size_t)kc * L * qp, rows_of(kc), qp, dq); };
 
+  // PIPE_LAST: the segment's start state, weighted end states summed by the whole workgroup in 16-byte
+  // pieces, four segments' reads in flight at a time, into the partial tiles' LDS as [DQK][64] columns and
+  // n.  Bound by the reads of the end states, which a head's segments share through their XCD's L2: B1 NH8
+  // S2011 DQK256 DV512 (4 segments of 7 chunks) 34.7 us for this launch, 41.2 with the segments of a head on
+  // different XCDs, and 36.5 + 7.8 for 8 chunks behind a combine kernel before.
+  constexpr int START_PITCH = 68;
+  if (MODE == PIPE_LAST) {
+    constexpr int NPC = DQK * 16 / NTHREADS;  // pieces per thread
+    f32x4 x[NPC];
+#pragma unroll
+    for (int u = 0; u < NPC; ++u) x[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float xn = 0.f, G = 0.f;
+    const int nrow = min(tid, dq - 1);
+    for (int s1 = seg - 1; s1 >= 0; s1 -= 4) {
+      f32x4 y[4][NPC];
+      float yn[4], wt[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int s = max(s1 - j, 0);  // past the first: read again, not added
+#pragma unroll
+        for (int u = 0; u < NPC; ++u) {
+          const int row = min((u * NTHREADS + tid) >> 4, dq - 1), c4 = tid & 15;  // rows past dq are not used
+          y[j][u] = *reinterpret_cast<const f32x4*>(sp.ec + s * cst + ((size_t)bh * dq + row) * DV + v0 + 4 * c4);
+        }
+        yn[j] = sp.en[s * nst + (size_t)bh * dq + nrow];
+        wt[j] = exp_(sp.em[(size_t)s * BNH + bh] + G - m_init);
+        G += sp.eg[(size_t)s * BNH + bh];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (s1 - j < 0) continue;
+#pragma unroll
+        for (int u = 0; u < NPC; ++u) x[u] += wt[j] * y[j][u];
+        xn = fmaf(wt[j], yn[j], xn);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NPC; ++u)
+      *reinterpret_cast<f32x4*>(hp + ((u * NTHREADS + tid) >> 4) * START_PITCH + 4 * (tid & 15)) = x[u];
+    if (tid < dq) hp[DQK * START_PITCH + tid] = xn;
+    __syncthreads();
+  }
+
   if (w < NSW) {
     // =====================================================================
     // state waves: rows [dw0, dw0 + DW) of C and n, stored as C e^{-G}, n e^{-G}
@@ -189,19 +243,31 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
       return dw0 + 32 * dt + 16 * (i >> 1) + 8 * hh + 4 * (i & 1) + (e & 3);
     };
     f32x16 acc[NDT][2];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int vt = 0; vt < 2; ++vt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          acc[dt][vt][e] = (ci && dw0 < dq) ? ci[((size_t)bh * dq + srow(dt, e)) * DV + v0 + 32 * vt + l32] : 0.f;
     // n of state row state_row(dw0, dt, l32): lane halves hh = 0, 1 sum the
     // tokens of their half of every 16-token k-step
     float nacc[NDT];
+    if (MODE == PIPE_LAST) {  // the start state composed in the partial tiles' LDS, above
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      nacc[dt] = (ni && hh == 0 && dw0 < dq) ? ni[(size_t)bh * dq + state_row(dw0, dt, l32)] : 0.f;
+      for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+        for (int vt = 0; vt < 2; ++vt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[dt][vt][e] = hp[srow(dt, e) * START_PITCH + 32 * vt + l32];
+        nacc[dt] = hh == 0 ? hp[DQK * START_PITCH + state_row(dw0, dt, l32)] : 0.f;
+      }
+      __syncthreads();  // read before the partials are written
+    } else {
+      const float *ci = seg == 0 ? a.c0 : nullptr, *ni = seg == 0 ? a.n0 : nullptr;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+        for (int vt = 0; vt < 2; ++vt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            acc[dt][vt][e] = (ci && dw0 < dq) ? ci[((size_t)bh * dq + srow(dt, e)) * DV + v0 + 32 * vt + l32] : 0.f;
+        nacc[dt] = (ni && hh == 0 && dw0 < dq) ? ni[(size_t)bh * dq + state_row(dw0, dt, l32)] : 0.f;
+      }
+    }
     // n entering chunk kc as two bf16 rows (hi, lo) of buffer kc & 1 (rows 2, 3 stay zero):
     // the fifth A tile of the output waves' S product
     auto store_nparts = [&](int buf) {
@@ -245,7 +311,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
         for (int s = 0; s < QKS; ++s)
           Qs[tt][s] = ld16s(rq, qs_off, (uint32_t)((32 * tt * qp + 16 * s) * 2));
     };
-    if (!STATES_ONLY) load_qs(kc0);
+    if (!states_only) load_qs(kc0);
     __syncthreads();  // B0: tiles, gate rows and n parts of the first chunk
 
     for (int kc = kc0; kc < kc1; ++kc) {
@@ -276,7 +342,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
 #pragma unroll
           for (int j = 0; j < 2; ++j) an[ks][j] = *reinterpret_cast<const s16x4*>(ab + 32 * ks + 8 * j);
       }
-      if (!STATES_ONLY) {
+      if (!states_only) {
         // Transposed product C^T Q^T per 32-column tile vt: lane (hh, l32) gets
         // columns 32 vt + 8i + 4hh + j of token 32 tt + l32.  The split of k-step
         // q+1 (VALU) is interleaved with the four MFMAs of k-step q, and the
@@ -376,7 +442,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
       }
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) nacc[dt] += nd[dt][0] + nd[dt][1];
-      if (!STATES_ONLY && kc + 1 < kc1) store_nparts((kc + 1) & 1);
+      if (!states_only && kc + 1 < kc1) store_nparts((kc + 1) & 1);
       __syncthreads();  // B1: the next chunk's tiles, gate rows and n parts are staged
     }
     // ---- final states (undo the deferred rescale)
@@ -404,6 +470,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
     // output waves: rows [16o, 16o + 16) of every chunk, the staging of K and V,
     // alpha' V one chunk ahead, and (wave 0 of the group) the gate rows
     // =====================================================================
+    if (MODE == PIPE_LAST) __syncthreads();  // the start state is read
     __builtin_amdgcn_s_setprio(2);
     const int t = tid - 64 * NSW;  // 0 .. NOT-1
     // ---- gate rows (output wave 0, one chunk ahead): row terms of the
@@ -415,6 +482,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
     // hi (64) | lo (64) in token order (the n update's operand).
     const float* preph = a.prep + (size_t)bh * NC * PREP_STRIDE;
     float gm = m_init, gG = 0.f;  // running m and G (every output wave runs the recurrence)
+    float gsum = 0.f;             // total log forget gate of the segment's chunks (PIPE_FIRST)
     auto prep_load = [&](int c, float (&pv)[5]) {
       const float* pc = preph + (size_t)c * PREP_STRIDE;
       pv[0] = pc[lane];
@@ -430,12 +498,15 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
       const float pg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pv[4]), 0));
       const float pamax = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pv[4]), 1));
       const float b = pv[0], av_ = pv[1], cmu = pv[2];
+      if (MODE == PIPE_FIRST) gsum += pg;
       const float m_next = fmaxf(pg + gm, pamax);
-      const float lg = pg + gm - m_next;  // log of this chunk's rescale of the state (<= 0)
+      // an empty state (-inf) that no token of a chunk enters stays empty
+      const bool empty = MODE == PIPE_FIRST && m_next == -INFINITY;
+      const float lg = empty ? 0.f : pg + gm - m_next;  // log of this chunk's rescale of the state (<= 0)
       float Gn = gG + lg;
       const bool renorm = Gn < E::RENORM;   // wave-uniform
       if (renorm) Gn = 0.f;
-      const float al = exp_(av_ - m_next - Gn);  // alpha' = exp(a_t - m') e^{-G}
+      const float al = empty ? 0.f : exp_(av_ - m_next - Gn);  // alpha' = exp(a_t - m') e^{-G}
       if (writer) {
         const float mb = b + gm;
         const float mc = fmaxf(mb, b + cmu);
@@ -531,7 +602,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
       };
       // prologue: the first chunk's tiles and gate rows, the second chunk's loads in flight
       load_kv(kc0);
-      if (!STATES_ONLY) load_q(kc0);
+      if (!states_only) load_q(kc0);
       prep_load(kc0, pv);
       alpha_v_regs(gate_rows(kc0, pv, o == 0));
       store_kv();
@@ -547,7 +618,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
         alpha_v_store();
         f32x4 Hmv[NVX];
         float qn = 0.f;
-        if (!STATES_ONLY) {
+        if (!states_only) {
           // S^T tiles over the whole DQK: A = K rows 16jt + r16, B = q rows; only the
           // causal j-tiles jt <= o (the rest are masked).  A fifth A tile holds n as
           // bf16 hi / lo rows (rows 2, 3 zero), so the same MFMAs give q.n.
@@ -621,7 +692,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
         // Q C of row 16o + r16, columns vcol_of(vq, 4g + e): sum of the four state waves'
         // partials (two 16-byte runs of 4 columns per tile pair)
         f32x4 Hqc[NVT];
-        if (!STATES_ONLY) {
+        if (!states_only) {
           const float* pr = hp + (16 * o + r16) * HP_PITCH;
 #pragma unroll
           for (int vq = 0; vq < NVT; ++vq) Hqc[vq] = *reinterpret_cast<const f32x4*>(pr + hp_col(8 * (vq >> 1) + 2 * g + (vq & 1)));
@@ -632,7 +703,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
               Hqc[vq] += *reinterpret_cast<const f32x4*>(pr + sw * 64 * HP_PITCH + hp_col(8 * (vq >> 1) + 2 * g + (vq & 1)));
         }
         if (kc + 1 < kc1) store_kv();
-        if (!STATES_ONLY) {
+        if (!states_only) {
           // this lane holds columns vcol_of(vq, 4g + e), i.e. the 8 consecutive
           // columns 32h + 8g .. +7 of tiles (2h, 2h+1); the row sum of M is element 0
           // of the fifth tile
@@ -660,6 +731,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
         prep_load(min(kc + 2, kc1 - 1), pv);
         __syncthreads();  // B1
       }
+      if (MODE == PIPE_FIRST && o == 0 && v0 == 0 && lane == 0) sp.eg[(size_t)seg * BNH + bh] = gsum;
     };
     switch (__builtin_amdgcn_readfirstlane(ws)) {
       case 0: out_wave(std::integral_constant<int, 0>{}); break;
@@ -670,28 +742,29 @@ __global__ __launch_bounds__(NTHREADS, 1) void chunkwise_pipe_kernel(MainArgs a)
   }
 }
 
-template <typename T, int DQK, bool STATES_ONLY>
-static int launch_one(unsigned nwg, hipStream_t st, const MainArgs& a) {
+template <typename T, int DQK, int MODE>
+static int launch_one(hipStream_t st, const MainArgs& a) {
   const size_t smem = Smem<DQK>::BYTES;
-  auto kern = a.strided ? chunkwise_pipe_kernel<T, DQK, STATES_ONLY, true> : chunkwise_pipe_kernel<T, DQK, STATES_ONLY, false>;
+  auto kern = a.strided ? chunkwise_pipe_kernel<T, DQK, MODE, true> : chunkwise_pipe_kernel<T, DQK, MODE, false>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess)
     return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_fwd: LDS attribute failed: %s", hipGetErrorString(e));
+  const unsigned nwg = (unsigned)(a.BNH * a.nvtile * a.sp.w);
   hipLaunchKernelGGL(kern, dim3(nwg), dim3(NTHREADS), smem, st, a);
   return XL_OK;
 }
 
-}  // namespace pipe
-
-template <typename T>
-static int pipe_launch_t(int DQK, bool states_only, unsigned nwg, hipStream_t st, const MainArgs& a) {
-  if (DQK == 256)
-    return states_only ? pipe::launch_one<T, 256, true>(nwg, st, a) : pipe::launch_one<T, 256, false>(nwg, st, a);
-  return states_only ? pipe::launch_one<T, 128, true>(nwg, st, a) : pipe::launch_one<T, 128, false>(nwg, st, a);
+template <typename T, int DQK>
+static int launch_mode(int mode, hipStream_t st, const MainArgs& a) {
+  if (mode == PIPE_FULL) return launch_one<T, DQK, PIPE_FULL>(st, a);
+  return mode == PIPE_FIRST ? launch_one<T, DQK, PIPE_FIRST>(st, a) : launch_one<T, DQK, PIPE_LAST>(st, a);
 }
 
-int pipe_launch(bool f16, int DQK, bool states_only, unsigned nwg, hipStream_t st, const MainArgs& a) {
-  return f16 ? pipe_launch_t<f16_t>(DQK, states_only, nwg, st, a) : pipe_launch_t<bf16_t>(DQK, states_only, nwg, st, a);
+}  // namespace pipe
+
+int pipe_launch(bool f16, int DQK, int mode, hipStream_t st, const MainArgs& a) {
+  if (DQK == 256) return f16 ? pipe::launch_mode<f16_t, 256>(mode, st, a) : pipe::launch_mode<bf16_t, 256>(mode, st, a);
+  return f16 ? pipe::launch_mode<f16_t, 128>(mode, st, a) : pipe::launch_mode<bf16_t, 128>(mode, st, a);
 }
 
 }  // namespace fused

@@ -155,6 +155,23 @@ struct SegArgs {
   float *ec, *en, *em;
 };
 
+// The pipelined kernel's split of the sequence (few heads: B * NH * DV / 64 workgroups leave CUs
+// idle) into 1 + w segments, segment 0 of n0 chunks and the others of n (the last one shorter), in two
+// launches of w segments each that both fill the chip:
+//   PIPE_FIRST: segment 0 complete (outputs and end state, from the caller's initial state) beside the
+//     end states alone of segments 1 .. w - 1, each from the empty state (C = n = 0, m = -inf); end
+//     states, m and total log forget gate of segment s in entry s of (ec, en, em, eg);
+//   PIPE_LAST: segments 1 .. w complete.  A workgroup forms its segment's start state from the end
+//     states before it: with G the sum of the later segments' eg, m = max_s(em_s + G_s) and
+//     X = sum_s exp(em_s + G_s - m) X_s (X = C, n): the inter-chunk recurrence of fw.py:115-133 over
+//     whole segments.
+// PIPE_FULL: one segment, no split.
+enum { PIPE_FULL = 0, PIPE_FIRST = 1, PIPE_LAST = 2 };
+struct SplitArgs {
+  int w, n0, n;
+  float *ec, *en, *em, *eg;
+};
+
 // LDS layout of one workgroup of the fused kernels (DQK 128 or 256, 64 DV columns).
 template <int DQK>
 struct Smem {
@@ -186,16 +203,17 @@ struct MainArgs {
   const float* prep;
   int S, NC, DV, BNH, nvtile;
   float qk_scale, eps;
-  SegArgs sg;
+  SegArgs sg;      // fused schedule
   int dq;  // q / k width in memory (DQK of the launch, or less: a multiple of DQK / 4)
   int NH;
   int strided;         // pipelined kernel: q, k, v at these strides (elements), else contiguous
   Strides qs, ks, vs;
+  SplitArgs sp;        // pipelined kernel
 };
 
-// The pipelined main kernel (chunkwise_pipe.hip): nwg workgroups of NTHREADS on stream st.
-// XL_OK or a negative XL_ERR_* code.
-int pipe_launch(bool f16, int DQK, bool states_only, unsigned nwg, hipStream_t st, const MainArgs& a);
+// The pipelined main kernel (chunkwise_pipe.hip), one of PIPE_*, on stream st.  XL_OK or a negative
+// XL_ERR_* code.
+int pipe_launch(bool f16, int DQK, int mode, hipStream_t st, const MainArgs& a);
 
 }  // namespace fused
 }  // namespace xl
