@@ -1,0 +1,21 @@
+"""The backward's fused path (bf16, DV 256 / 512) where its launches change form: n and m in blocks of 64 chunks
+(more than 64, one past a block), both row widths of the paired scans (64 rows up to 256 workgroups of 128, 128
+beyond), and workgroup counts that are no multiple of 8 (the XCD grouping).  Bars of test_gpu_chunkwise_bwd.py."""
+
+import pytest
+import torch
+
+from test_gpu_chunkwise_bwd import _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 1, 64 * 65, 128, 256),    # one chunk past a block of 64
+                                           (1, 2, 64 * 64, 64, 256),     # exactly a block
+                                           (3, 6, 64, 128, 512),         # 288 workgroups of 128 rows
+                                           (1, 16, 128, 128, 512),       # 256: the last that takes 64 rows
+                                           (1, 9, 192, 256, 512),        # 288, two row slices a state
+                                           (1, 1, 128, 128, 256)])
+@pytest.mark.parametrize("states", [False, True])
+def test_forms(gpu_case, B, NH, S, DQK, DV, states):
+    _run(B, NH, S, DQK, DV, 64, torch.bfloat16, states, states, seed=S + DQK + B)

@@ -27,10 +27,13 @@
 // Workspace (float32, each region 256-byte aligned): the entering states C, n, m
 // [BNH][NC](...), the final state, m_comb and the divisor [BNH][S], dC
 // [BNH][NC + 1][DQK][DV] (index k: the gradient of the state after chunk k - 1;
-// 0 is dC_initial), the dF partials [BNH][S][ceil(DQK/64)] and the dI partials
+// 0 is dC_initial), the chunks' own contributions to n [BNH][NC][DQK] and b - m_comb [BNH][S] (fused path),
+// the dF partials [BNH][S][ceil(DQK/64)] and the dI partials
 // [BNH][S][ceil(DV/64)].  On the path of the fused bf16 dV / dQ / dK pass the C and
 // dC states are kept as their upper 24 bits (pack24 below), in the first three
-// quarters of their regions.
+// quarters of their regions, n and m entering every chunk come from a pass of their own
+// (bw_nloc_kernel, bw_nscan_kernel), the stats pass follows, and both state recurrences (1, 3)
+// run in one launch (bw_scan_pair_kernel).
 #include "chunkwise.h"
 #include "mfma_bf16.h"
 
@@ -94,7 +97,7 @@ __device__ __forceinline__ float xor_lane(float x, int lane) {
 }
 
 struct BwLayout {
-  size_t Cst, nst, mst, cfin, nfin, mfin, vm, vn, dC, dfp, dip, gprep, total;
+  size_t Cst, nst, mst, cfin, nfin, mfin, vm, vn, dC, dfp, dip, gprep, nloc, rb, total;
 };
 
 constexpr int GP_STRIDE = kChunkGatePrefix;  // floats per chunk of the scans' gate prefix
@@ -123,6 +126,8 @@ BwLayout bw_layout(int B, int NH, int S, int DQK, int DV, int L) {
   o.dfp = take(BNH * S * ndt);
   o.dip = take(BNH * S * nvt);
   o.gprep = take(BNH * NC * GP_STRIDE);
+  o.nloc = take(BNH * NC * DQK);
+  o.rb = take(BNH * S);
   o.total = off;
   return o;
 }
@@ -620,33 +625,64 @@ __global__ __launch_bounds__(BW_THREADS) void bw_dqk_kernel(const TQ* __restrict
 // each workgroup sums itself (a plain reduction over contiguous partials).
 constexpr int GSEG = 1024;
 
-template <typename TG>
+// NDT, NVT: the partials per token, 0 where only known at run time.  Every load is issued before the first
+// sum (the partials of a thread's 4 tokens and 16-byte pieces of the later segments': with one load at a
+// time the pass took 25 us at B2 NH8 S4096 DQK256 DV512, so 9).
+template <typename TG, int NDT, int NVT>
 __global__ __launch_bounds__(256) void bw_gates_kernel(const TG* __restrict__ fg, const float* __restrict__ dfp,
                                                        const float* __restrict__ dip, TG* __restrict__ di,
-                                                       TG* __restrict__ df, int S, int ndt, int nvt) {
+                                                       TG* __restrict__ df, int S, int ndt_arg, int nvt_arg) {
   __shared__ float s_wave[4], s_red[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int ndt = NDT ? NDT : ndt_arg, nvt = NVT ? NVT : nvt_arg;
   const int nseg = (S + GSEG - 1) / GSEG;
   const int bh = blockIdx.x / nseg, sg = blockIdx.x - bh * nseg;
   const size_t base = (size_t)bh * S;
   const int t0 = sg * GSEG, t1 = min(S, t0 + GSEG);
+  // this thread's tokens t0 + 4 tid + u (past t1: token t1 - 1 read again, not used)
+  float pd[4][NDT ? NDT : 1], pi[4][NVT ? NVT : 1], fv[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const size_t t = base + min(t0 + 4 * tid + u, t1 - 1);
+    if constexpr (NDT > 0) {
+#pragma unroll
+      for (int j = 0; j < NDT; ++j) pd[u][j] = dfp[t * NDT + j];
+    }
+    if constexpr (NVT > 0) {
+#pragma unroll
+      for (int j = 0; j < NVT; ++j) pi[u][j] = dip[t * NVT + j];
+    }
+    fv[u] = to_f32(fg[t]);
+  }
   // total of the later segments' partials
   float c = 0.f;
   const float* later = dfp + (base + t1) * ndt;
   const size_t nl = (size_t)(S - t1) * ndt;
-  for (size_t e = tid; e < nl; e += 256) c += later[e];
-  // this thread's tokens t0 + 4 tid + u
-  float x[4], fv[4];
+  if ((((base + t1) * ndt | nl) & 3) == 0) {
+    const f32x4* l4 = reinterpret_cast<const f32x4*>(later);
+    const size_t n4 = nl / 4;
+    f32x4 cs[8] = {};
+    for (size_t e = tid; e < n4; e += 8 * 256)
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (e + 256 * u < n4) cs[u] += l4[e + 256 * u];
+#pragma unroll
+    for (int u = 4; u > 0; u >>= 1)
+#pragma unroll
+      for (int j = 0; j < u; ++j) cs[j] += cs[j + u];
+    c = (cs[0][0] + cs[0][1]) + (cs[0][2] + cs[0][3]);
+  } else {
+    for (size_t e = tid; e < nl; e += 256) c += later[e];
+  }
+  float x[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int t = t0 + 4 * tid + u;
     float a = 0.f, sd = 0.f;
-    fv[u] = 0.f;
     if (t < t1) {
-      for (int j = 0; j < ndt; ++j) a += dfp[(base + t) * ndt + j];
-      for (int j = 0; j < nvt; ++j) sd += dip[(base + t) * nvt + j];
+      for (int j = 0; j < ndt; ++j) a += NDT ? pd[u][j] : dfp[(base + t) * ndt + j];
+      for (int j = 0; j < nvt; ++j) sd += NVT ? pi[u][j] : dip[(base + t) * nvt + j];
       di[base + t] = from_f32<TG>(sd);
-      fv[u] = to_f32(fg[base + t]);
     }
     x[u] = a;
   }
@@ -903,8 +939,9 @@ __global__ __launch_bounds__(256) void bw_stats_bf16_kernel(const bf16_t* __rest
                                                              const TG* __restrict__ ig, const TG* __restrict__ fg,
                                                              const float* __restrict__ nst,
                                                              const float* __restrict__ mst, float* __restrict__ vm,
-                                                             float* __restrict__ vn, float* __restrict__ gp, int NC,
-                                                             float qk_scale, float eps) {
+                                                             float* __restrict__ vn, float* __restrict__ gp,
+                                                             float* __restrict__ rb, int NC, float qk_scale,
+                                                             float eps) {
   constexpr int L = 64, DQK = 64 * NRT;
   constexpr int KP = DQK + 16;               // bf16 per staged K row (2 DQK + 32 bytes)
   constexpr int PR = DQK / 8, NP = L * PR / 256;  // 16-byte pieces per row, per thread
@@ -980,9 +1017,8 @@ __global__ __launch_bounds__(256) void bw_stats_bf16_kernel(const bf16_t* __rest
       vm[row0 + i] = smc[i];
       vn[row0 + i] = dv;
       if (gp) {  // the dC scan's per-token factors (bw.py:92-101): b - m_comb and qk_scale / divisor
-        float* g = gp + sidx * GP_STRIDE;
-        g[64 + i] = sb[i] - smc[i];
-        g[132 + i] = qk_scale / dv;
+        rb[row0 + i] = sb[i] - smc[i];
+        gp[sidx * GP_STRIDE + 132 + i] = qk_scale / dv;
       }
     }
   }
@@ -1028,28 +1064,39 @@ __global__ __launch_bounds__(256) void bw_gate_prep_kernel(const TG* __restrict_
 constexpr int SB_YP = SC_V + 16;  // bf16 per staged hi / lo row (160 bytes)
 constexpr int SST_P = SC_V + 4;  // floats per LDS row of a state store (conflict-free 16-byte writes and reads)
 
-// two workgroups per CU (at most 256 registers per lane): the scans are bound by their state
-// stores, and two workgroups keep more of them in flight
-template <typename TG, int L, int NRT, bool REV, bool PK>
-__global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
-    const bf16_t* __restrict__ X, const bf16_t* __restrict__ Y, const TG* __restrict__ ig,
-    const TG* __restrict__ fg, const float* __restrict__ gp, const float* __restrict__ s0,
-    const float* __restrict__ n0, const float* __restrict__ m0, const float* __restrict__ vm,
-    const float* __restrict__ vn, float* __restrict__ Sst, float* __restrict__ nst, float* __restrict__ mst,
-    float* __restrict__ sfin, float* __restrict__ nfin, float* __restrict__ mfin, float* __restrict__ s_init, int NC,
-    int DQKf, int DV, int nvt, float qk_scale) {
+// What one scan works on.
+template <typename TG>
+struct ScanArgs {
+  const bf16_t *X, *Y;
+  const TG *ig, *fg;
+  const float *gp, *rb, *s0, *n0, *m0, *vm, *vn;
+  float *Sst, *nst, *mst, *sfin, *nfin, *mfin, *s_init;
+};
+
+template <int L, int NRT>
+struct ScanSmem {
+  bf16_t sX[L * (64 * NRT + 16)];
+  bf16_t sYh[L * SB_YP];
+  bf16_t sYl[L * SB_YP];
+  float sSt[4][16 * NRT * SST_P];  // per wave: its state rows, for the stores
+};
+
+// Workgroup `blk` of the scan (logical: a head's column tiles and row slices in a row).  WITH_N: the first
+// column tile's workgroups carry n and write m (the fused path takes both from bw_nscan_kernel).
+template <typename TG, int L, int NRT, bool REV, bool PK, bool WITH_N>
+__device__ __forceinline__ void scan_bf16(const ScanArgs<TG>& A, ScanSmem<L, NRT>& sm, int blk, int NC, int DQKf, int DV,
+                                          int nvt, float qk_scale) {
   static_assert(L % 32 == 0, "32-token MFMA steps");
   constexpr int DQK = 64 * NRT;  // state rows of this workgroup
   constexpr int XP = DQK + 16;   // bf16 per staged X row
   constexpr int PRX = DQK / 8, NX = L * PRX, NXP = (NX + 255) / 256;
   constexpr int PRY = SC_V / 8, NY = L * PRY, NYP = (NY + 255) / 256;
-  __shared__ __attribute__((aligned(16))) bf16_t sX[L * XP];
-  __shared__ __attribute__((aligned(16))) bf16_t sYh[L * SB_YP];
-  __shared__ __attribute__((aligned(16))) bf16_t sYl[L * SB_YP];
-  __shared__ __attribute__((aligned(16))) float sSt[4][16 * NRT * SST_P];  // per wave: its state rows, for the stores
+  const bf16_t *X = A.X, *Y = A.Y;
+  const float *gp = A.gp, *s0 = A.s0, *n0 = A.n0, *m0 = A.m0, *vm = A.vm, *vn = A.vn;
+  float *Sst = A.Sst, *nst = A.nst, *mst = A.mst, *sfin = A.sfin, *nfin = A.nfin, *mfin = A.mfin, *s_init = A.s_init;
+  bf16_t *sX = sm.sX, *sYh = sm.sYh, *sYl = sm.sYl;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, r = lane & 15;
   const int nrs = DQKf / DQK;
-  const int blk = xcd_contiguous(blockIdx.x, gridDim.x);
   const int bhv = blk / nrs, rs = blk - bhv * nrs;
   const int bh = bhv / nvt, vt = bhv - bh * nvt, v0 = vt * SC_V;
   const int d_off = rs * DQK;
@@ -1072,7 +1119,7 @@ __global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
   // piece would be 64 bytes, and the stores, sent to L2 as 64-byte requests, capped the scans'
   // write rate at about 2.8 TB/s.  Only this wave touches its rows: no barrier.
   // With PK the per-chunk states (slots) go out as pack24 (12-byte pieces of 192-byte block rows).
-  float* const st_w = sSt[w];
+  float* const st_w = sm.sSt[w];
   auto store_state = [&](float* dst, bool packed) {
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt)
@@ -1098,7 +1145,7 @@ __global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
   // accumulator tile per row tile, whose A operand is columns 64.. of the staged hi rows: coef_t
   // hi in column 64, lo in column 65, zeros after; n[row 16 rt + r] = elements 0 + 1 of lane
   // (0, r)
-  const bool owns_n = !REV && vt == 0;  // workgroup-uniform
+  const bool owns_n = WITH_N && !REV && vt == 0;  // workgroup-uniform
   f32x4 accN[NRT];
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt)
@@ -1136,7 +1183,7 @@ __global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
       const int t = (u * 256 + tid) / PRY;
       if (NY % 256 == 0 || t < L) {
         if (REV && PK) {  // b - m_comb and qk_scale / divisor, from the stats pass
-          ga[u] = gb[64 + t];
+          ga[u] = A.rb[t0 + t];
           gvn[u] = gb[132 + t];
         } else {
           ga[u] = REV ? gb[t] : gb[64 + t];
@@ -1210,7 +1257,7 @@ __global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
     __syncthreads();
     store_state(slot_ptr(slot), PK);
     if (owns_n) store_n(nst + sidx * DQKf);
-    if (!REV && vt == 0 && rs == 0 && tid == 0) mst[sidx] = m_in;
+    if (WITH_N && !REV && vt == 0 && rs == 0 && tid == 0) mst[sidx] = m_in;
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
 #pragma unroll
@@ -1249,11 +1296,152 @@ __global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(
   if (!REV) {  // the final state (the forward's last states may not be asked for)
     if (sfin) store_state(sfin + (size_t)bh * DQKf * DV, false);
     if (owns_n && nfin) store_n(nfin + (size_t)bh * DQKf);
-    if (vt == 0 && rs == 0 && tid == 0 && mfin) mfin[bh] = m;
+    if (WITH_N && vt == 0 && rs == 0 && tid == 0 && mfin) mfin[bh] = m;
   } else {
     store_state(slot_ptr(0), PK);
     if (s_init) store_state(s_init + (size_t)bh * DQKf * DV, false);
   }
+}
+
+// two workgroups per CU (at most 256 registers per lane): the scans are bound by their state
+// stores, and two workgroups keep more of them in flight
+template <typename TG, int L, int NRT, bool REV>
+__global__ __launch_bounds__(256, 2) void bw_scan_bf16_kernel(ScanArgs<TG> A, int NC, int DQKf, int DV, int nvt,
+                                                              float qk_scale) {
+  __shared__ __attribute__((aligned(16))) ScanSmem<L, NRT> sm;
+  scan_bf16<TG, L, NRT, REV, false, true>(A, sm, xcd_contiguous(blockIdx.x, gridDim.x), NC, DQKf, DV, nvt, qk_scale);
+}
+
+// Both scans of the fused path in one launch, pack24 states: a chunk of a scan is a chain (stage, store
+// the state, update) of ~2.3 us that leaves half of a CU's two workgroups idle when the heads are few, and
+// the two scans do not depend on each other once n and m come from bw_nscan_kernel.  Groups of 8 blocks
+// (one per XCD) alternate between the directions, so each XCD and CU gets both.  One after the other / in one
+// launch: 294 / 243 us at B2 NH8 S4096 DQK256 DV512, 64 / 25 at B2 NH8 S1024 DQK128 DV256 (64-row slices); the
+// whole backward at B1 NH4 S8192 DQK256 DV512 628 / 389, at B4 NH8 S8192 (each scan fills the chip) 2118 / 2115.
+template <typename TG, int NRT>
+__global__ __launch_bounds__(256, 2) void bw_scan_pair_kernel(ScanArgs<TG> F, ScanArgs<TG> R, int NC, int DQKf, int DV,
+                                                              int nvt, float qk_scale) {
+  __shared__ __attribute__((aligned(16))) ScanSmem<64, NRT> sm;
+  const int G = gridDim.x >> 1, b = blockIdx.x;
+  bool rev = b >= G;
+  int i = rev ? b - G : b;
+  if ((G & 7) == 0) {
+    rev = (b >> 3) & 1;
+    i = ((b >> 4) << 3) | (b & 7);
+  }
+  i = xcd_contiguous(i, G);
+  if (rev)
+    scan_bf16<TG, 64, NRT, true, true, false>(R, sm, i, NC, DQKf, DV, nvt, qk_scale);
+  else
+    scan_bf16<TG, 64, NRT, false, true, false>(F, sm, i, NC, DQKf, DV, nvt, qk_scale);
+}
+
+// The gate prefix of a chunk (bw_gate_prep_kernel's, one wave) and the chunk's own contribution to n,
+// nloc[d] = sum_t exp(a_t - max a) K[t][d] in float32, all chunks at once: with them n and m entering
+// every chunk need no pass over the states.  One workgroup of 256 threads per chunk: thread (token
+// group, 16-byte piece) sums its tokens' rows (all loads first), the groups meet in LDS.
+template <typename TG, int NRT>
+__global__ __launch_bounds__(256) void bw_nloc_kernel(const bf16_t* __restrict__ k, const TG* __restrict__ ig,
+                                                      const TG* __restrict__ fg, float* __restrict__ gp,
+                                                      float* __restrict__ nloc) {
+  constexpr int L = 64, DQK = 64 * NRT, PR = DQK / 8, TGR = 256 / PR, NT = L / TGR;
+  __shared__ float sco[L];
+  __shared__ float spart[TGR][DQK + 4];
+  const int tid = threadIdx.x, c = blockIdx.x;
+  const int piece = tid % PR, tg = tid / PR;
+  const size_t t0 = (size_t)c * L;
+  u32x4 kv[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+    kv[u] = *reinterpret_cast<const u32x4*>(k + (t0 + tg + TGR * u) * DQK + 8 * piece);
+  if (tid < 64) {
+    const float b = wave_incl_sum(logsigmoid(to_f32(fg[t0 + tid])), tid);
+    const float gl = lane_of(b, L - 1);
+    const float a = gl - b + to_f32(ig[t0 + tid]);
+    const float amax = wave_max_rows(a);
+    float* p = gp + (size_t)c * GP_STRIDE;
+    p[tid] = b;
+    p[64 + tid] = a;
+    if (tid == 0) {
+      p[128] = gl;
+      p[129] = amax;
+    }
+    sco[tid] = amax == -INFINITY ? 0.f : expf(a - amax);  // no token enters
+  }
+  __syncthreads();
+  float x[8] = {};
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    const float co = sco[tg + TGR * u];
+    Piece16<bf16_t> pc;
+    pc.raw = kv[u];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = fmaf(co, to_f32(pc.v[e]), x[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) spart[tg][8 * piece + e] = x[e];
+  __syncthreads();
+  if (tid < DQK) {
+    float n = 0.f;
+#pragma unroll
+    for (int t = 0; t < TGR; ++t) n += spart[t][tid];
+    nloc[(size_t)c * DQK + tid] = n;
+  }
+}
+
+// n and m entering every chunk, and m after the last: n' = exp(gl + m - m') n + exp(max a - m') nloc,
+// m' = max(gl + m, max a) (fw.py:115-133; m in the scans' own order of operations).  One wave per (head,
+// 64 columns), 64 chunks at a time: only m runs chunk by chunk through the lanes' gl and max a (lane =
+// chunk), both factors of every chunk are formed at once, and a chunk then is one multiply and one
+// multiply-add on n.  10.0 us at 64 chunks of 16 heads against 15.1 with the factors formed in the chain.
+__global__ __launch_bounds__(64) void bw_nscan_kernel(const float* __restrict__ gp, const float* __restrict__ nloc,
+                                                      const float* __restrict__ n0, const float* __restrict__ m0,
+                                                      float* __restrict__ nst, float* __restrict__ mst,
+                                                      float* __restrict__ mfin, int NC, int DQK) {
+  constexpr int NB = 16;
+  const int lane = threadIdx.x, ncol = DQK >> 6, bh = blockIdx.x / ncol, d = (blockIdx.x - bh * ncol) * 64 + lane;
+  const bool first = blockIdx.x == bh * ncol;
+  float n = n0 ? n0[(size_t)bh * DQK + d] : 0.f, m = m0 ? m0[bh] : 0.f;
+  for (int c0 = 0; c0 < NC; c0 += 64) {
+    const int nc = min(64, NC - c0);
+    const size_t at = (size_t)bh * NC + c0;
+    const float* g = gp + (at + min(lane, nc - 1)) * GP_STRIDE;
+    const float gl = g[128], am = g[129];
+    const float* nl = nloc + at * DQK + d;
+    float x[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) x[u] = nl[(size_t)min(u, nc - 1) * DQK];
+    float m_in = m, m_out = m;  // entering and leaving chunk c0 + lane
+#pragma unroll 4
+    for (int u = 0; u < nc; ++u) {
+      const float mn = fmaxf(lane_of(gl, u) + m, lane_of(am, u));
+      if (lane == u) {
+        m_in = m;
+        m_out = mn;
+      }
+      m = mn;
+    }
+    // (loops kept rolled: straight-line code for 64 chunks spent its time on instruction fetches)
+    const float decay = expf(gl + m_in - m_out), w = expf(am - m_out);
+    if (first && lane < nc) mst[at + lane] = m_in;
+    float* ns = nst + at * DQK + d;
+#pragma unroll 1
+    for (int b = 0; b * NB < nc; ++b) {
+      float y[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) y[u] = nl[(size_t)min((b + 1) * NB + u, nc - 1) * DQK];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        const int c = b * NB + u;
+        if (c < nc) {
+          ns[(size_t)c * DQK] = n;
+          n = lane_of(decay, c) * n + lane_of(w, c) * x[u];
+        }
+        x[u] = y[u];
+      }
+    }
+  }
+  if (first && lane == 0) mfin[bh] = m;
 }
 
 // ---------------------------------------------------------------- launchers
@@ -2329,31 +2517,53 @@ __global__ __launch_bounds__(FV_THREADS) void bw_dvqk_bf16_kernel(
 }
 
 
-template <typename TQ, typename TG, int L, bool REV, bool PK = false>
+template <typename TQ, typename TG, int L, bool REV>
 int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, const float* gp, const float* s0,
                 const float* n0, const float* m0, const float* vm, const float* vn, float* Sst, float* nst, float* mst,
                 float* sfin, float* nfin, float* mfin, float* s_init, int BNH, int NC, int DV, float qk_scale,
                 hipStream_t st) {
   const int nvt = DV / SC_V;
+  const char* who = REV ? "xl_mlstm_chunkwise_bwd(dC scan)" : "xl_mlstm_chunkwise_bwd(states scan)";
   // 128 state rows per workgroup (64 for DQK 64): two workgroups share a DQK 256 state, so
   // the chunk-sequential scan keeps two waves on every SIMD
-  auto go = [&](auto kern, size_t smem, int nrs, auto... gprep) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess)
-      return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_bwd: LDS attribute failed: %s", hipGetErrorString(e));
-    hipLaunchKernelGGL(kern, dim3((unsigned)(BNH * nvt * nrs)), dim3(256), smem, st, X, Y, ig, fg, gprep..., s0, n0, m0,
-                       vm, vn, Sst, nst, mst, sfin, nfin, mfin, s_init, NC, DQK, DV, nvt, qk_scale);
-    return check_launch(REV ? "xl_mlstm_chunkwise_bwd(dC scan)" : "xl_mlstm_chunkwise_bwd(states scan)");
-  };
   if constexpr (std::is_same<TQ, bf16_t>::value && L % 32 == 0) {  // bf16 operands, static LDS, gate prefix in gp
-    if (DQK == 64) return go(bw_scan_bf16_kernel<TG, L, 1, REV, PK>, 0, 1, gp);
-    return go(bw_scan_bf16_kernel<TG, L, 2, REV, PK>, 0, DQK / 128, gp);
+    const ScanArgs<TG> a = {X, Y, ig, fg, gp, nullptr, s0, n0, m0, vm, vn, Sst, nst, mst, sfin, nfin, mfin, s_init};
+    const dim3 grid((unsigned)(BNH * nvt * (DQK == 64 ? 1 : DQK / 128)));
+    if (DQK == 64)
+      hipLaunchKernelGGL((bw_scan_bf16_kernel<TG, L, 1, REV>), grid, dim3(256), 0, st, a, NC, DQK, DV, nvt, qk_scale);
+    else
+      hipLaunchKernelGGL((bw_scan_bf16_kernel<TG, L, 2, REV>), grid, dim3(256), 0, st, a, NC, DQK, DV, nvt, qk_scale);
+    return check_launch(who);
   } else {
-    static_assert(!PK, "pack24 states come from the bf16 scans only");
+    auto go = [&](auto kern, size_t smem, int nrs) {
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+      if (e != hipSuccess)
+        return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_bwd: LDS attribute failed: %s", hipGetErrorString(e));
+      hipLaunchKernelGGL(kern, dim3((unsigned)(BNH * nvt * nrs)), dim3(256), smem, st, X, Y, ig, fg, s0, n0, m0, vm, vn,
+                         Sst, nst, mst, sfin, nfin, mfin, s_init, NC, DQK, DV, nvt, qk_scale);
+      return check_launch(who);
+    };
     if (DQK == 64) return go(bw_scan_kernel<TQ, TG, L, 1, REV>, scan_smem<TQ, L>(1), 1);
     return go(bw_scan_kernel<TQ, TG, L, 2, REV>, scan_smem<TQ, L>(2), DQK / 128);
   }
 }
+
+template <typename TG>
+int launch_gates(const TG* fg, const float* dfp, const float* dip, void* di, void* df, int BNH, int S, int ndt, int nvt,
+                 hipStream_t st) {
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(BNH * ((S + GSEG - 1) / GSEG))), dim3(256), 0, st, fg, dfp, dip, (TG*)di,
+                       (TG*)df, S, ndt, nvt);
+    return check_launch("xl_mlstm_chunkwise_bwd(gates)");
+  };
+  if (ndt == 4 && nvt == 8) return go(bw_gates_kernel<TG, 4, 8>);
+  if (ndt == 2 && nvt == 4) return go(bw_gates_kernel<TG, 2, 4>);
+  return go(bw_gates_kernel<TG, 0, 0>);
+}
+
+// 128-row workgroups of both scans together up to which they take 64 rows each instead: below one per CU a
+// scan's time is its chain (2.3 us a chunk at 128 rows, 1.5 at 64)
+constexpr int SCAN_FEW = 256;
 
 template <typename TQ, typename TG, int L>
 int bw_launch(const BwArgs& A, const BwLayout& lay) {
@@ -2364,7 +2574,8 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
   float *Cst = (float*)(ws + lay.Cst), *nst = (float*)(ws + lay.nst), *mst = (float*)(ws + lay.mst);
   float *cfin = (float*)(ws + lay.cfin), *nfin = (float*)(ws + lay.nfin), *mfin = (float*)(ws + lay.mfin);
   float *vm = (float*)(ws + lay.vm), *vn = (float*)(ws + lay.vn), *dC = (float*)(ws + lay.dC);
-  float *dfp = (float*)(ws + lay.dfp), *dip = (float*)(ws + lay.dip), *gpr = (float*)(ws + lay.gprep);
+  float *dfp = (float*)(ws + lay.dfp), *dip = (float*)(ws + lay.dip), *gpr = (float*)(ws + lay.gprep),
+        *nlc = (float*)(ws + lay.nloc), *rbw = (float*)(ws + lay.rb);
   hipStream_t s = (hipStream_t)F.stream;
   const TQ *q = (const TQ*)F.q, *k = (const TQ*)F.k, *v = (const TQ*)F.v, *dh = (const TQ*)A.dh;
   const TG *ig = (const TG*)F.i, *fg = (const TG*)F.f;
@@ -2374,18 +2585,26 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
   constexpr bool fused_types = std::is_same<TQ, bf16_t>::value && L == 64;
   const bool fused_dvqk = fused_types && scan_mfma && (F.DV == 256 || F.DV == 512);
   int rc = XL_OK;
-  // the bf16 chunk scans take every chunk's gate prefix from gpr
+  if constexpr (fused_types) {
+    if (fused_dvqk) {  // n and m entering every chunk without the states: the stats pass then runs before the scans
+      const dim3 grid((unsigned)(BNH * NC));
+      switch (F.DQK) {
+        case 64: hipLaunchKernelGGL((bw_nloc_kernel<TG, 1>), grid, dim3(256), 0, s, k, ig, fg, gpr, nlc); break;
+        case 128: hipLaunchKernelGGL((bw_nloc_kernel<TG, 2>), grid, dim3(256), 0, s, k, ig, fg, gpr, nlc); break;
+        default: hipLaunchKernelGGL((bw_nloc_kernel<TG, 4>), grid, dim3(256), 0, s, k, ig, fg, gpr, nlc); break;
+      }
+      hipLaunchKernelGGL(bw_nscan_kernel, dim3((unsigned)(BNH * (F.DQK / 64))), dim3(64), 0, s, gpr, nlc, F.n0, F.m0, nst,
+                         mst, mfin, NC, F.DQK);
+      rc = check_launch("xl_mlstm_chunkwise_bwd(n scan)");
+    }
+  }
+  // otherwise the bf16 chunk scans take every chunk's gate prefix from gpr
   if constexpr (std::is_same<TQ, bf16_t>::value && L % 32 == 0) {
-    if (scan_mfma) {
+    if (scan_mfma && !fused_dvqk) {
       hipLaunchKernelGGL((bw_gate_prep_kernel<TG, L>), dim3((unsigned)((BNH * NC + 3) / 4)), dim3(256), 0, s, ig, fg,
                          gpr, BNH * NC);
       if ((rc = check_launch("xl_mlstm_chunkwise_bwd(gate prefix)"))) return rc;
     }
-  }
-  if constexpr (fused_types) {
-    if (fused_dvqk)
-      rc = launch_scan<TQ, TG, L, false, true>(F.DQK, k, v, ig, fg, gpr, F.c0, F.n0, F.m0, nullptr, nullptr, Cst, nst,
-                                               mst, cfin, nfin, mfin, nullptr, BNH, NC, F.DV, F.qk_scale, s);
   }
   if (!fused_dvqk)
     rc = scan_mfma ? launch_scan<TQ, TG, L, false>(F.DQK, k, v, ig, fg, gpr, F.c0, F.n0, F.m0, nullptr, nullptr, Cst,
@@ -2397,9 +2616,9 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
     stats_mfma = F.DQK == 64 || F.DQK == 128 || F.DQK == 256;
     const dim3 grid((unsigned)(BNH * NC));
     switch (stats_mfma ? F.DQK : 0) {
-      case 64: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 1>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, NC, F.qk_scale, F.eps); break;
-      case 128: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 2>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, NC, F.qk_scale, F.eps); break;
-      case 256: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 4>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, NC, F.qk_scale, F.eps); break;
+      case 64: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 1>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, rbw, NC, F.qk_scale, F.eps); break;
+      case 128: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 2>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, rbw, NC, F.qk_scale, F.eps); break;
+      case 256: hipLaunchKernelGGL((bw_stats_bf16_kernel<TG, 4>), grid, dim3(256), 0, s, q, k, ig, fg, nst, mst, vm, vn, fused_dvqk ? gpr : nullptr, rbw, NC, F.qk_scale, F.eps); break;
       default: break;
     }
   }
@@ -2408,9 +2627,21 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
                        nst, mst, vm, vn, NC, F.DQK, F.qk_scale, F.eps);
   if ((rc = check_launch("xl_mlstm_chunkwise_bwd(stats)"))) return rc;
   if constexpr (fused_types) {
-    if (fused_dvqk)
-      rc = launch_scan<TQ, TG, L, true, true>(F.DQK, q, dh, ig, fg, gpr, A.dc_last, nullptr, nullptr, vm, vn, dC,
-                                              nullptr, mst, nullptr, nullptr, mfin, A.dc0, BNH, NC, F.DV, F.qk_scale, s);
+    if (fused_dvqk) {
+      const ScanArgs<TG> fw = {k, v, ig, fg, gpr, nullptr, F.c0, nullptr, F.m0, nullptr, nullptr, Cst, nullptr, nullptr,
+                               nullptr, nullptr, nullptr, nullptr};
+      const ScanArgs<TG> rv = {q, dh, ig, fg, gpr, rbw, A.dc_last, nullptr, nullptr, nullptr, nullptr, dC, nullptr, mst,
+                               nullptr, nullptr, mfin, A.dc0};
+      // 128 state rows per workgroup; 64 where the two scans would otherwise leave CUs without one
+      const int nv = F.DV / SC_V, wide = 2 * BNH * nv * (F.DQK / 128);
+      if (F.DQK == 64 || wide <= SCAN_FEW)
+        hipLaunchKernelGGL((bw_scan_pair_kernel<TG, 1>), dim3((unsigned)(2 * BNH * nv * (F.DQK / 64))), dim3(256), 0, s, fw,
+                           rv, NC, F.DQK, F.DV, nv, F.qk_scale);
+      else
+        hipLaunchKernelGGL((bw_scan_pair_kernel<TG, 2>), dim3((unsigned)wide), dim3(256), 0, s, fw, rv, NC, F.DQK, F.DV, nv,
+                           F.qk_scale);
+      rc = check_launch("xl_mlstm_chunkwise_bwd(scans)");
+    }
   }
   if (fused_dvqk) {
   } else if (scan_mfma) {
@@ -2441,9 +2672,7 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
         default: rc = wide ? go(bw_dvqk_bf16_kernel<TG, 4, 8>, dvqk_smem<4>()) : go(bw_dvqk_bf16_kernel<TG, 4, 4>, dvqk_smem<4>()); break;
       }
       if (rc) return rc;
-      hipLaunchKernelGGL((bw_gates_kernel<TG>), dim3((unsigned)(BNH * ((F.S + GSEG - 1) / GSEG))), dim3(256), 0, s,
-                         fg, dfp, dip, (TG*)A.di, (TG*)A.df, F.S, ndt, nvt);
-      return check_launch("xl_mlstm_chunkwise_bwd(gates)");
+      return launch_gates<TG>(fg, dfp, dip, A.di, A.df, BNH, F.S, ndt, nvt, s);
     }
   }
   // dV and dQ/dK on the matrix cores for 16-bit operands, 64-token chunks and whole 64-wide tiles
@@ -2494,9 +2723,7 @@ int bw_launch(const BwArgs& A, const BwLayout& lay) {
                        F.qk_scale);
   }
   if ((rc = check_launch("xl_mlstm_chunkwise_bwd(dQ, dK)"))) return rc;
-  hipLaunchKernelGGL((bw_gates_kernel<TG>), dim3((unsigned)(BNH * ((F.S + GSEG - 1) / GSEG))), dim3(256), 0, s, fg,
-                     dfp, dip, (TG*)A.di, (TG*)A.df, F.S, ndt, nvt);
-  return check_launch("xl_mlstm_chunkwise_bwd(gates)");
+  return launch_gates<TG>(fg, dfp, dip, A.di, A.df, BNH, F.S, ndt, nvt, s);
 }
 
 template <typename TQ, typename TG>
