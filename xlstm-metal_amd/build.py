@@ -1,11 +1,12 @@
-"""Builds libxlstm_hip.so for gfx950 from csrc/*.hip (in-tree, no JIT cache).
+"""Builds libxlstm_hip.so for gfx950 from csrc/*.hip and libxlstm_torch.so, the torch operators around it,
+from csrc/torch_ops.cpp (in-tree, no JIT cache).
 
     python xlstm-metal_amd/build.py            # build (always recompiles)
     python xlstm-metal_amd/build.py --jobs 8
 
-Objects go to xlstm-metal_amd/_build/, the library to
-xlstm-metal_amd/xlstm_hip/lib/libxlstm_hip.so (git-ignored; it travels to
-the GPU box with the tree).
+Objects go to xlstm-metal_amd/_build/, the libraries to
+xlstm-metal_amd/xlstm_hip/lib/ (git-ignored; they travel to the GPU box with
+the tree).
 """
 
 from __future__ import annotations
@@ -22,6 +23,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "xlstm_hip", "lib")
 LIB = os.path.join(LIBDIR, "libxlstm_hip.so")
+OPS_LIB = os.path.join(LIBDIR, "libxlstm_torch.so")
+OPS_SRC = os.path.join(CSRC, "torch_ops.cpp")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 ARCH = "gfx950"
 
@@ -62,21 +65,50 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_ops() -> str:
+    """Host code only: g++ against torch's headers (torch's own libraries are in the process already)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    obj = os.path.join(BUILD, "torch_ops.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{INCLUDE}",
+           *[f"-isystem{d}" for d in include_paths("cuda")], "-isystem/opt/rocm/include", "-c", OPS_SRC, "-o", obj]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{res.stderr}")
+    return obj
+
+
+def _link_ops(obj: str) -> None:
+    import torch
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = OPS_LIB + ".tmp"
+    cmd = ["g++", "-shared", "-fPIC", "-o", tmp, obj, f"-L{LIBDIR}", "-lxlstm_hip", "-Wl,-rpath,$ORIGIN", f"-L{tlib}",
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,--no-as-needed"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link failed: {' '.join(cmd)}\n{res.stderr}")
+    os.replace(tmp, OPS_LIB)
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> str:
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     srcs = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
     jobs = jobs or min(8, len(srcs))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        ops = ex.submit(_compile_ops)
         objs = list(ex.map(_compile, srcs))
+        ops_obj = ops.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{res.stderr}")
     os.replace(tmp, LIB)
+    _link_ops(ops_obj)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources")
+        print(f"built {LIB} from {len(srcs)} sources and {OPS_LIB}")
     return LIB
 
 

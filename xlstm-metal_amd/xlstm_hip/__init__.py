@@ -5,8 +5,9 @@ mLSTM prefill and its custom backward, recurrent decode step and sequence, sLSTM
 the sLSTM layer's causal conv1d + SiLU and per-head GroupNorm, the mLSTM
 output cell's multi-head RMSNorm x sigmoid(o), soft_cap and the logit
 projection with its soft-cap epilogue,
-each a ``torch.library`` op (``xlstm_hip::*``) calling hand-written HIP
-kernels in ``lib/libxlstm_hip.so`` through a C-ABI.
+each a ``torch.library`` op (``xlstm_hip::*``, native kernels in
+``lib/libxlstm_torch.so``) calling hand-written HIP kernels in
+``lib/libxlstm_hip.so`` through a C-ABI.
 """
 
 from . import _lib

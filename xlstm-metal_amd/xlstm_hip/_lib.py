@@ -15,6 +15,9 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libxlstm_hip.so")
 
+# the native operator kernels (csrc/torch_ops.cpp)
+OPS_PATH = os.path.join(os.path.dirname(LIB_PATH), "libxlstm_torch.so")
+
 XL_DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 XL_ERRORS = {-1: "invalid argument", -2: "unsupported", -3: "workspace", -4: "launch"}
 
@@ -60,6 +63,19 @@ _lib = None
 _lock = threading.Lock()
 
 
+def missing(path: str = OPS_PATH) -> str:
+    return (f"xlstm_hip: HIP library not found at {path}; build it with "
+            "`python xlstm-metal_amd/build.py` (there is no CPU fallback)")
+
+
+def load_ops() -> bool:
+    """Loads the operator kernels; False where they have not been built (the ops then raise)."""
+    if not (os.path.exists(OPS_PATH) and os.path.exists(LIB_PATH)):
+        return False
+    torch.ops.load_library(OPS_PATH)
+    return True
+
+
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Loads the library once and declares every signature; raises if absent."""
     global _lib
@@ -67,9 +83,7 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         if _lib is not None:
             return _lib
         if not os.path.exists(path):
-            raise RuntimeError(
-                f"xlstm_hip: HIP library not found at {path}; build it with "
-                "`python xlstm-metal_amd/build.py` (there is no CPU fallback)")
+            raise RuntimeError(missing(path))
         lib = ctypes.CDLL(path)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)

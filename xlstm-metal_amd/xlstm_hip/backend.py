@@ -13,7 +13,7 @@ raise ``NotImplementedError``.
 from __future__ import annotations
 
 from dataclasses import dataclass
-from functools import partial
+from functools import lru_cache, partial
 from typing import Callable, Literal
 
 import torch
@@ -79,8 +79,13 @@ def _fused_takes_any_length(q, k, v) -> bool:
     ragged last chunk)."""
     if not (q.dtype == k.dtype == v.dtype and q.dtype in (torch.bfloat16, torch.float16)):
         return False
-    B, NH, S, DQK = q.shape
-    return chunkwise_workspace_bytes(B, NH, S, DQK, v.shape[-1], 64, q.dtype, algo="pipelined") > 0
+    return _pipelined_heads(q.shape[-1], v.shape[-1], q.dtype)
+
+
+@lru_cache(maxsize=64)
+def _pipelined_heads(DQK: int, DV: int, dtype) -> bool:
+    """The library's answer, which depends on the head widths and the dtype only."""
+    return chunkwise_workspace_bytes(1, 1, 64, DQK, DV, 64, dtype, algo="pipelined") > 0
 
 
 def wrap_chunkwise__arbitrary_sequence_length(mlstm_chunkwise_kernel, mlstm_sequence_kernel, mlstm_step_kernel, q,
