@@ -19,3 +19,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("states", [False, True])
 def test_forms(gpu_case, B, NH, S, DQK, DV, states):
     _run(B, NH, S, DQK, DV, 64, torch.bfloat16, states, states, seed=S + DQK + B)
+
+
+@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 2, 192, 256, 128), (2, 8, 64, 128, 1024), (3, 6, 64, 128, 1024)])
+def test_float32_row_slices(gpu_case, B, NH, S, DQK, DV):
+    """The float32 scans with 64 rows a workgroup (up to 256 workgroups of 128 rows: 4 slices of a state, exactly
+    256) and 128 (288), forward and backward."""
+    _run(B, NH, S, DQK, DV, 64, torch.float32, True, True, seed=DV)

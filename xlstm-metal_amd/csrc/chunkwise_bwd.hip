@@ -2517,6 +2517,10 @@ __global__ __launch_bounds__(FV_THREADS) void bw_dvqk_bf16_kernel(
 }
 
 
+// 128-row workgroups (of both scans together in bw_scan_pair_kernel) up to which they take 64 rows each instead: below one per CU a
+// scan's time is its chain (2.3 us a chunk at 128 rows, 1.5 at 64)
+constexpr int SCAN_FEW = 256;
+
 template <typename TQ, typename TG, int L, bool REV>
 int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, const float* gp, const float* s0,
                 const float* n0, const float* m0, const float* vm, const float* vn, float* Sst, float* nst, float* mst,
@@ -2543,7 +2547,10 @@ int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, c
                          Sst, nst, mst, sfin, nfin, mfin, s_init, NC, DQK, DV, nvt, qk_scale);
       return check_launch(who);
     };
-    if (DQK == 64) return go(bw_scan_kernel<TQ, TG, L, 1, REV>, scan_smem<TQ, L>(1), 1);
+    // 64 rows where 128 would leave CUs without a workgroup or with one: a chunk is then a chain of staging,
+    // stores and MFMAs on few waves (float32 B1 NH8 S1024 DQK256 DV512: 79.6 -> 58.5 us)
+    if (DQK == 64 || BNH * nvt * (DQK / 128) <= SCAN_FEW)
+      return go(bw_scan_kernel<TQ, TG, L, 1, REV>, scan_smem<TQ, L>(1), DQK / 64);
     return go(bw_scan_kernel<TQ, TG, L, 2, REV>, scan_smem<TQ, L>(2), DQK / 128);
   }
 }
@@ -2560,10 +2567,6 @@ int launch_gates(const TG* fg, const float* dfp, const float* dip, void* di, voi
   if (ndt == 2 && nvt == 4) return go(bw_gates_kernel<TG, 2, 4>);
   return go(bw_gates_kernel<TG, 0, 0>);
 }
-
-// 128-row workgroups of both scans together up to which they take 64 rows each instead: below one per CU a
-// scan's time is its chain (2.3 us a chunk at 128 rows, 1.5 at 64)
-constexpr int SCAN_FEW = 256;
 
 template <typename TQ, typename TG, int L>
 int bw_launch(const BwArgs& A, const BwLayout& lay) {
