@@ -1,5 +1,5 @@
 """The backward's fused path (bf16, DV 256 / 512) where its launches change form: n and m in blocks of 64 chunks
-(more than 64, one past a block), both row widths of the paired scans (64 rows up to 256 workgroups of 128, 128
+(more than 64, one past a block), both row widths of the paired scans (64 rows up to 128 workgroups of 128, 128
 beyond), and workgroup counts that are no multiple of 8 (the XCD grouping).  Bars of test_gpu_chunkwise_bwd.py."""
 
 import pytest
@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 1, 64 * 65, 128, 256),    # one chunk past a block of 64
                                            (1, 2, 64 * 64, 64, 256),     # exactly a block
                                            (3, 6, 64, 128, 512),         # 288 workgroups of 128 rows
-                                           (1, 16, 128, 128, 512),       # 256: the last that takes 64 rows
+                                           (1, 8, 128, 128, 512),        # 128: the last that takes 64 rows
+                                           (1, 9, 128, 128, 512),        # 144: the first that takes 128
                                            (1, 9, 192, 256, 512),        # 288, two row slices a state
                                            (1, 1, 128, 128, 256)])
 @pytest.mark.parametrize("states", [False, True])
@@ -21,8 +22,8 @@ def test_forms(gpu_case, B, NH, S, DQK, DV, states):
     _run(B, NH, S, DQK, DV, 64, torch.bfloat16, states, states, seed=S + DQK + B)
 
 
-@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 2, 192, 256, 128), (2, 8, 64, 128, 1024), (3, 6, 64, 128, 1024)])
+@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 2, 192, 256, 128), (1, 8, 64, 128, 1024), (1, 9, 64, 128, 1024)])
 def test_float32_row_slices(gpu_case, B, NH, S, DQK, DV):
-    """The float32 scans with 64 rows a workgroup (up to 256 workgroups of 128 rows: 4 slices of a state, exactly
-    256) and 128 (288), forward and backward."""
+    """The float32 scans with 64 rows a workgroup (up to 128 workgroups of 128 rows: 4 slices of a state, exactly
+    128) and 128 (144), forward and backward."""
     _run(B, NH, S, DQK, DV, 64, torch.float32, True, True, seed=DV)

@@ -2517,9 +2517,12 @@ __global__ __launch_bounds__(FV_THREADS) void bw_dvqk_bf16_kernel(
 }
 
 
-// 128-row workgroups (of both scans together in bw_scan_pair_kernel) up to which they take 64 rows each instead: below one per CU a
-// scan's time is its chain (2.3 us a chunk at 128 rows, 1.5 at 64)
-constexpr int SCAN_FEW = 256;
+// 128-row workgroups (of both scans together in bw_scan_pair_kernel) up to which they take 64 rows each
+// instead, so that every CU has one: a scan's time then is its chain, 2.3 us a chunk at 128 rows, 1.5 at 64.
+// The whole backward with 64 / 128 rows: 128 workgroups 67 / 73 us (B2 NH8 S1024 DQK128 DV256) and 387 / 406
+// (B1 NH4 S8192 DQK256 DV512), 192 workgroups 163 / 153, 256 workgroups 722 / 667; the paired scans at 512
+// 305 / 244.
+constexpr int SCAN_FEW = 128;
 
 template <typename TQ, typename TG, int L, bool REV>
 int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, const float* gp, const float* s0,
@@ -2547,8 +2550,8 @@ int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, c
                          Sst, nst, mst, sfin, nfin, mfin, s_init, NC, DQK, DV, nvt, qk_scale);
       return check_launch(who);
     };
-    // 64 rows where 128 would leave CUs without a workgroup or with one: a chunk is then a chain of staging,
-    // stores and MFMAs on few waves (float32 B1 NH8 S1024 DQK256 DV512: 79.6 -> 58.5 us)
+    // 64 rows where 128 would leave CUs without a workgroup: a chunk is a chain of staging, stores and MFMAs
+    // on few waves (float32 B1 NH8 S1024 DQK256 DV512: 79.6 -> 58.5 us)
     if (DQK == 64 || BNH * nvt * (DQK / 128) <= SCAN_FEW)
       return go(bw_scan_kernel<TQ, TG, L, 1, REV>, scan_smem<TQ, L>(1), DQK / 64);
     return go(bw_scan_kernel<TQ, TG, L, 2, REV>, scan_smem<TQ, L>(2), DQK / 128);
