@@ -620,12 +620,12 @@ def bwd_flops(B, NH, S, DQK, DV, L):
     return 2.0 * B * NH * NC * (5 * L * DQK * DV + 4 * L * L * DQK + 2 * L * L * DV)
 
 
-FUSED_PATH = ["states scan", "stats", "dC scan", "dV, dQ, dK", "gate gradients"]
+FUSED_PATH = ["gate prefix, n terms", "n and m", "stats", "state scans", "dV, dQ, dK", "gate gradients"]
 
 
 def bwd_bytes(B, NH, S, DQK, DV, L, esz=2):
     """HBM bytes of this design's backward on the path config 2 takes (bf16, 64-token chunks, DV 256
-    or 512): the algorithmic bytes of its five launches (bwd_kernel_bytes), with the per-chunk
+    or 512): the algorithmic bytes of its six launches (bwd_kernel_bytes), with the per-chunk
     states C and dC materialised once each (bw.py: matC_states recomputed, matDeltaC_states) in
     the 24-bit packed form, written by the scans and read once by the fused dV / dQ / dK pass."""
     kb = bwd_kernel_bytes(B, NH, S, DQK, DV, L, esz, st_esz=3)
@@ -640,9 +640,10 @@ def bwd_io_bytes(B, NH, S, DQK, DV, esz=2):
 
 
 BWD_KERNELS = {  # kernel-name key -> short name, for the trace / counter summaries of the backward
-    "bw_scan_bf16_kernel<xl::bf16_t, 64, 2, false, true>": "states scan",
+    "bw_nloc_kernel": "gate prefix, n terms",
+    "bw_nscan_kernel": "n and m",
     "bw_stats_bf16_kernel": "stats",
-    "bw_scan_bf16_kernel<xl::bf16_t, 64, 2, true, true>": "dC scan",
+    "bw_scan_pair_kernel": "state scans",
     "bw_dv_bf16_kernel": "dV",
     "bw_dqk_bf16_kernel": "dQ, dK",
     "bw_dvqk_bf16_kernel": "dV, dQ, dK",
@@ -658,9 +659,15 @@ def bwd_kernel_bytes(B, NH, S, DQK, DV, L, esz=2, st_esz=4):
     st = NC * DQK * DV * st_esz
     g = 2 * S * esz  # i, f
     return {
-        "states scan": BNH * (S * (DQK + DV) * esz + g + st + NC * (DQK + 1) * 4 + (DQK * DV + DQK + 1) * 4),
-        "stats": BNH * (2 * S * DQK * esz + g + NC * (DQK + 1) * 4 + 2 * S * 4),
-        "dC scan": BNH * (S * (DQK + DV) * esz + g + 2 * S * 4 + NC * 4 + DQK * DV * 4 + st + DQK * DV * st_esz),
+        # k and the gates in; b, a, the chunk's decay and max a, and its own contribution to n out
+        "gate prefix, n terms": BNH * (S * DQK * esz + g + NC * (2 * L + 2 + DQK) * 4),
+        "n and m": BNH * (NC * (2 + DQK) * 4 + NC * (DQK + 1) * 4),
+        # and the dC scan's per-token factors out
+        "stats": BNH * (2 * S * DQK * esz + g + NC * (DQK + 1) * 4 + 4 * S * 4),
+        # both recurrences: k v / q dH in with the chunks' decays and two per-token rows each, the
+        # states out, dC_last in, C_last / dC_initial out
+        "state scans": BNH * (2 * S * (DQK + DV) * esz + 4 * S * 4 + 2 * st + 2 * DQK * DV * 4
+                              + DQK * DV * st_esz),
         "dV": BNH * (2 * S * DQK * esz + 2 * S * DV * esz + st + g + 2 * S * 4 + S * DV * esz + S * nvt * 4),
         "dQ, dK": BNH * (2 * S * DQK * esz + 2 * S * DV * esz + 2 * st + g + 2 * S * 4 + 2 * S * DQK * esz
                          + S * ndt * 4),
@@ -873,17 +880,17 @@ def summarize_trace(trace_dir, headline_calls):
         sn = short(name)
         per.setdefault(sn, []).append(us)
         # a timed call: flush fill, then the call's gate prep, then this kernel
-        if (sn.startswith(PREFILL_KERNEL + "<bf16_t, 256, false>") and "gate_prep_kernel" in prev[1][0]
+        if (sn.startswith(PREFILL_KERNEL + "<bf16_t, 256, 0, false>") and "gate_prep_kernel" in prev[1][0]
                 and "FillFunctor<float>" in prev[0][0] and prev[0][1] >= 40.0):
             head.append(us)
         prev = [prev[1], (name, us)]
     warm, head = head[:PATTERN_WARM_CALLS], head[PATTERN_WARM_CALLS:PATTERN_WARM_CALLS + headline_calls]
     print("| kernel | calls | mean us | min us | max us |\n|---|---|---|---|---|")
     if head:
-        print(f"| {PREFILL_KERNEL}<bf16_t, 256, false>, the {len(head)} timed cfg2 headline calls (after the cache "
+        print(f"| {PREFILL_KERNEL}<bf16_t, 256, 0, false>, the {len(head)} timed cfg2 headline calls (after the cache "
               f"flush) | {len(head)} | {statistics.mean(head):.1f} | {min(head):.1f} | {max(head):.1f} |")
     if warm:
-        print(f"| {PREFILL_KERNEL}<bf16_t, 256, false>, the headline's {len(warm)} untimed (flush, call) pairs before "
+        print(f"| {PREFILL_KERNEL}<bf16_t, 256, 0, false>, the headline's {len(warm)} untimed (flush, call) pairs before "
               f"them | {len(warm)} | {statistics.mean(warm):.1f} | {min(warm):.1f} | {max(warm):.1f} |")
     for name, ts in sorted(per.items(), key=lambda kv: -sum(kv[1])):
         print(f"| {name} | {len(ts)} | {statistics.mean(ts):.1f} | {min(ts):.1f} | {max(ts):.1f} |")

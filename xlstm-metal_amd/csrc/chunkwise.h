@@ -60,8 +60,8 @@ int chunkwise_states_pass(const ChunkwiseArgs& a, float* Cst, float* nst, float*
 // kChunkGatePrefix floats per chunk of every head.
 int chunkwise_states_mfma(const ChunkwiseArgs& a, float* Cst, float* nst, float* mst, float* gprep);
 // floats per chunk of the bf16 chunk scans' gate prefix: b[64], a[64], the chunk's log-decay, max a,
-// two spare, and (the backward's fused path, written by its stats pass over a) the dC scan's
-// per-token b - m_comb in place of a and qk_scale / divisor [64]
+// two spare, and (the backward's fused path, written by its stats pass) the dC scan's per-token
+// qk_scale / divisor [64]
 constexpr int kChunkGatePrefix = 196;
 
 // The single-pass algorithms.  fused_supported() says whether a shape/dtype is covered by the

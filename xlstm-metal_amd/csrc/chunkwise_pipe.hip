@@ -37,8 +37,9 @@
 // tile is single-buffered: K and V of the next chunk are written only in
 // phase B, after the last reads of the current ones (the state waves took
 // their K^T operands in phase A).  The deferred forget rescale (state stored
-// as C e^{-G}, renormalised when G < -30), the ragged last chunk, the
-// sequence segments and the XCD-aware grid are those of the fused kernel.
+// as C e^{-G}, renormalised when G < -30), the ragged last chunk and
+// the XCD-aware grid are those of the fused kernel; the sequence segments are
+// its own (PIPE_FIRST, PIPE_LAST).
 #include "fused_common.h"
 
 #include <type_traits>
