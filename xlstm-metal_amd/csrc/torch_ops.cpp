@@ -293,20 +293,27 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> mlstm_chunkwise_bwd(
 // unchanged (ops._PAD_I, ops._PAD_F; test_state_preserving_padding).
 constexpr double kPadI = -3.0e4, kPadF = 30.0;
 
+// Sizes stay symbolic from here to the backward's results: a traced training step then serves every
+// sequence length (the kernels above get plain integers from the dispatcher).
 FourTensors call_chunkwise(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& i, const Tensor& f,
-                           const OptTensor& c0, const OptTensor& n0, const OptTensor& m0, double qk_scale, int64_t chunk,
-                           double eps, bool ret, int64_t algo) {
+                           const OptTensor& c0, const OptTensor& n0, const OptTensor& m0, double qk_scale,
+                           c10::SymInt chunk, double eps, bool ret, c10::SymInt algo) {
   static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("xlstm_hip::mlstm_chunkwise", "")
-                             .typed<decltype(mlstm_chunkwise)>();
+                             .typed<decltype(call_chunkwise)>();
   at::AutoDispatchBelowADInplaceOrView below;
   return op.call(q, k, v, i, f, c0, n0, m0, qk_scale, chunk, eps, ret, algo);
 }
 
+using SixTensors = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+using ChunkwiseBwd = SixTensors(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const OptTensor&,
+                                const OptTensor&, const OptTensor&, const Tensor&, const OptTensor&, double, c10::SymInt,
+                                double);
+
 struct ChunkwiseFn : public torch::autograd::Function<ChunkwiseFn> {
   static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k,
                                                 const Tensor& v, const Tensor& i, const Tensor& f, const OptTensor& c0,
-                                                const OptTensor& n0, const OptTensor& m0, double qk_scale, int64_t chunk,
-                                                double eps, bool ret, int64_t algo) {
+                                                const OptTensor& n0, const OptTensor& m0, double qk_scale,
+                                                c10::SymInt chunk, double eps, bool ret, c10::SymInt algo) {
     ctx->save_for_backward({q, k, v, i, f, c0.value_or(Tensor()), n0.value_or(Tensor()), m0.value_or(Tensor())});
     ctx->saved_data["qk_scale"] = qk_scale;
     ctx->saved_data["chunk"] = chunk;
@@ -320,27 +327,28 @@ struct ChunkwiseFn : public torch::autograd::Function<ChunkwiseFn> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
     static const auto bwd = c10::Dispatcher::singleton().findSchemaOrThrow("xlstm_hip::mlstm_chunkwise_bwd", "")
-                                .typed<decltype(mlstm_chunkwise_bwd)>();
+                                .typed<ChunkwiseBwd>();
     auto saved = ctx->get_saved_variables();
     Tensor q = saved[0], k = saved[1], v = saved[2], i = saved[3], f = saved[4];
     const Tensor c0 = saved[5], n0 = saved[6], m0 = saved[7];
     auto given = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
-    const int64_t S = q.size(2);
+    const c10::SymInt S = q.sym_size(2);
     Tensor dh = grads[0];
-    if (!dh.defined()) dh = at::zeros({q.size(0), q.size(1), S, v.size(3)}, q.options());
+    if (!dh.defined()) dh = at::zeros_symint({q.sym_size(0), q.sym_size(1), S, v.sym_size(3)}, q.options());
     const OptTensor dcl = ctx->saved_data["ret"].toBool() ? given(grads[1]) : OptTensor();
-    int64_t L = ctx->saved_data["chunk"].toInt();
+    int64_t L = ctx->saved_data["chunk"].toSymInt().guard_int(__FILE__, __LINE__);
     if ((L != 16 && L != 32 && L != 64) || S % L != 0) L = 64;
-    const int64_t pad = (L - S % L) % L;
-    if (pad) {
-      for (Tensor* t : {&q, &k, &v, &dh}) *t = at::constant_pad_nd(*t, {0, 0, 0, pad});
-      i = at::constant_pad_nd(i, {0, pad}, kPadI);
-      f = at::constant_pad_nd(f, {0, pad}, kPadF);
+    const bool ragged = S % L != 0;
+    if (ragged) {
+      const c10::SymInt pad = L - S % L;
+      for (Tensor* t : {&q, &k, &v, &dh}) *t = at::constant_pad_nd_symint(*t, {0, 0, 0, pad});
+      i = at::constant_pad_nd_symint(i, {0, pad}, kPadI);
+      f = at::constant_pad_nd_symint(f, {0, pad}, kPadF);
     }
     auto [dq, dk, dv, di, df, dc0] = bwd.call(q, k, v, i, f, given(c0), given(n0), given(m0), dh, dcl,
                                               ctx->saved_data["qk_scale"].toDouble(), L, ctx->saved_data["eps"].toDouble());
-    if (pad)
-      for (Tensor* t : {&dq, &dk, &dv, &di, &df}) *t = t->slice(2, 0, S).contiguous();
+    if (ragged)
+      for (Tensor* t : {&dq, &dk, &dv, &di, &df}) *t = t->slice_symint(2, 0, S).contiguous();
     const Tensor none;
     return {dq,
             dk,
@@ -360,7 +368,7 @@ struct ChunkwiseFn : public torch::autograd::Function<ChunkwiseFn> {
 
 FourTensors mlstm_chunkwise_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& i, const Tensor& f,
                                      const OptTensor& c0, const OptTensor& n0, const OptTensor& m0, double qk_scale,
-                                     int64_t chunk, double eps, bool ret, int64_t algo) {
+                                     c10::SymInt chunk, double eps, bool ret, c10::SymInt algo) {
   auto wants = [](const Tensor* t) { return t && t->defined() && (t->requires_grad() || t->_fw_grad(0).defined()); };
   bool any = false;
   for (const Tensor* t : {&q, &k, &v, &i, &f, opt(c0), opt(n0), opt(m0)}) any = any || wants(t);

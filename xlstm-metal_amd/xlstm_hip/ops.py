@@ -34,12 +34,12 @@ _SCHEMAS = {
     "mlstm_step_": ("(Tensor q, Tensor k, Tensor v, Tensor i, Tensor f, Tensor(a!) c, Tensor n, Tensor m, "
                    "float eps, float qk_scale) -> (Tensor, Tensor, Tensor)"),
     "mlstm_chunkwise": ("(Tensor q, Tensor k, Tensor v, Tensor i, Tensor f, Tensor? c0, Tensor? n0, Tensor? m0, "
-                       "float qk_scale, int chunk_size, float eps, bool return_last_states, int algo) -> "
+                       "float qk_scale, SymInt chunk_size, float eps, bool return_last_states, SymInt algo) -> "
                        "(Tensor, Tensor, Tensor, Tensor)"),
     # the reference's custom backward (mlstm_chunkwise_bw, bw.py:198-352): dq, dk, dv (q's dtype), di, df
     # (the gates' dtype) and dc0 (float32; an empty placeholder without initial states)
     "mlstm_chunkwise_bwd": ("(Tensor q, Tensor k, Tensor v, Tensor i, Tensor f, Tensor? c0, Tensor? n0, Tensor? m0, "
-                           "Tensor dh, Tensor? dc_last, float qk_scale, int chunk_size, float eps) -> (Tensor, "
+                           "Tensor dh, Tensor? dc_last, float qk_scale, SymInt chunk_size, float eps) -> (Tensor, "
                            "Tensor, Tensor, Tensor, Tensor, Tensor)"),
     "mlstm_sequence": ("(Tensor q, Tensor k, Tensor v, Tensor i, Tensor f, Tensor? c0, Tensor? n0, Tensor? m0, "
                       "float qk_scale, float eps, bool return_last_states) -> (Tensor, Tensor, Tensor, Tensor)"),
@@ -50,13 +50,13 @@ _SCHEMAS = {
     # h and the last states packed as one flat tensor [c | n | m] (state_views)
     "slstm_sequence": ("(Tensor z, Tensor i, Tensor f, Tensor o, Tensor? c0, Tensor? n0, Tensor? m0, float eps) "
                       "-> (Tensor, Tensor)"),
-    "causal_conv1d": ("(Tensor x, Tensor weight, Tensor? bias, int act) -> Tensor"),
-    "group_norm": ("(Tensor x, int num_groups, Tensor? weight, Tensor? bias, float eps) -> Tensor"),
+    "causal_conv1d": ("(Tensor x, Tensor weight, Tensor? bias, SymInt act) -> Tensor"),
+    "group_norm": ("(Tensor x, SymInt num_groups, Tensor? weight, Tensor? bias, float eps) -> Tensor"),
     "mh_rmsnorm_gate": ("(Tensor h, Tensor? weight, Tensor? o_preact, bool heads_first, float eps) -> Tensor"),
-    "gate_proj_softcap": ("(Tensor x, Tensor weight, Tensor? bias, float cap, int cap_rounding=0) -> Tensor"),
+    "gate_proj_softcap": ("(Tensor x, Tensor weight, Tensor? bias, float cap, SymInt cap_rounding=0) -> Tensor"),
     # gate_proj_softcap for two projections of one input [B, S, D], their weights not stacked; the
     # outputs [B, S, G], or [B, G, S] with heads_first
-    "gate_proj2_softcap": ("(Tensor x, Tensor w1, Tensor? b1, Tensor w2, Tensor? b2, float cap, int cap_rounding, "
+    "gate_proj2_softcap": ("(Tensor x, Tensor w1, Tensor? b1, Tensor w2, Tensor? b2, float cap, SymInt cap_rounding, "
                           "bool heads_first) -> (Tensor, Tensor)"),
     # soft_cap(x weight^T, cap) for at most LM_HEAD_MAX_ROWS rows
     "lm_head_softcap": ("(Tensor x, Tensor weight, float cap) -> Tensor"),
