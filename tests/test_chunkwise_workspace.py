@@ -1,0 +1,23 @@
+"""The single-pass forward's workspace (no GPU): each schedule asks for its own per-segment states and no more."""
+
+import pytest
+import torch
+
+
+def _segments(B, NH, S, DQK, DV, algo):
+    """The workspace past the gate prep, and the bytes of one segment's states (C, n, m and, in the pipelined
+    schedule, the total log forget gate)."""
+    from xlstm_hip.ops import chunkwise_workspace_bytes
+    total = chunkwise_workspace_bytes(B, NH, S, DQK, DV, 64, torch.bfloat16, algo=algo)
+    prep = -(-B * NH * -(-S // 64) * 1280 // 256) * 256
+    return total - prep, B * NH * (DQK * DV + DQK + (2 if algo == "pipelined" else 1)) * 4
+
+
+# one column tile (15 end states at most), the 7B head's prompt, no split
+@pytest.mark.parametrize("B,NH,S,DQK,DV,most", [(1, 1, 64 * 130, 128, 64, 15), (1, 8, 2011, 256, 512, 4),
+                                                (1, 2, 2048, 256, 128, 15), (4, 8, 8192, 256, 512, 0)])
+def test_pipelined_workspace_holds_end_states_only(B, NH, S, DQK, DV, most):
+    states, one = _segments(B, NH, S, DQK, DV, "pipelined")
+    assert states <= most * one + 256
+    fused, one = _segments(B, NH, S, DQK, DV, "fused")
+    assert fused <= 2 * 15 * one + 512

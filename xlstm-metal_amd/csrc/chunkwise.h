@@ -68,12 +68,12 @@ constexpr int kChunkGatePrefix = 196;
 // pipelined schedule (pipelined: bf16 or f16 q/k/v) or the fused one (bf16 only), and why not,
 // in `why`, when it is not.
 bool chunkwise_fused_supported(const ChunkwiseArgs& a, const char** why, bool pipelined);
-// Workspace of the fused algorithm: the gate prep (1280 bytes per 64-token chunk of every
-// head) and, when the sequence is split into segments (few heads), two sets of per-segment
-// states.  max_segments 1 disables the split.
+// Workspace of the single-pass algorithms: the gate prep (1280 bytes per 64-token chunk of every
+// head) and, when the sequence is split into segments (few heads), per-segment states: one set, the
+// end states, in the pipelined schedule's own split, two (end and start states) in the fused one's.
+// max_segments 1 disables the split.
 constexpr int kChunkwiseMaxSegments = 16;
-size_t chunkwise_fused_workspace(int B, int NH, int S, int DQK, int DV, int max_segments);
-int chunkwise_fused_segments(int B, int NH, int S, int DQK, int DV, int max_segments);
+size_t chunkwise_fused_workspace(int B, int NH, int S, int DQK, int DV, int max_segments, bool pipelined);
 int chunkwise_fused(const ChunkwiseArgs& a);
 
 }  // namespace xl

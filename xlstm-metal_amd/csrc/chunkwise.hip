@@ -64,8 +64,9 @@ extern "C" size_t xl_mlstm_chunkwise_workspace_size(int B, int NH, int S, int DQ
   a.dtype_qkv = dtype_qkv; a.dtype_gates = dtype_qkv;
   int chosen = XL_CHUNKWISE_TWO_PASS;
   if (pick(a, algo, &chosen) != XL_OK) return 0;
-  return single_pass(chosen) ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments)
-                                     : chunkwise_two_pass_workspace(B, NH, S, DQK, DV, L);
+  return single_pass(chosen) ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments,
+                                                         chosen == XL_CHUNKWISE_PIPELINED)
+                             : chunkwise_two_pass_workspace(B, NH, S, DQK, DV, L);
 }
 
 extern "C" int xl_mlstm_chunkwise_algo(int B, int NH, int S, int DQK, int DV, int L, int dtype_qkv, int algo) {
@@ -102,7 +103,7 @@ static int forward(ChunkwiseArgs& a, int algo) {
   if (rc) return rc;
   const bool fused = single_pass(chosen);
   a.pipelined = chosen == XL_CHUNKWISE_PIPELINED;
-  const size_t need = fused ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments)
+  const size_t need = fused ? chunkwise_fused_workspace(B, NH, S, DQK, DV, kChunkwiseMaxSegments, a.pipelined)
                             : chunkwise_two_pass_workspace(B, NH, S, DQK, DV, L);
   if (!a.workspace || a.workspace_bytes < need)
     return set_error(XL_ERR_WORKSPACE, "xl_mlstm_chunkwise_fwd: %s workspace needs %zu bytes, got %zu",

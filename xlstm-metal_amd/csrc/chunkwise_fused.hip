@@ -793,12 +793,10 @@ static int launch(const ChunkwiseArgs& A) {
                      (const TG*)A.f, prep, total, NC, A.S);
   if (A.pipelined) return launch_pipe(A, DQK, prep);
   const size_t smem = Smem<DQK>::BYTES;
-  {
-    for (auto kern : {chunkwise_fused_kernel<DQK, false>, chunkwise_fused_kernel<DQK, true>}) {
-      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-      if (e != hipSuccess)
-        return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_fwd: LDS attribute failed: %s", hipGetErrorString(e));
-    }
+  for (auto kern : {chunkwise_fused_kernel<DQK, false>, chunkwise_fused_kernel<DQK, true>}) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess)
+      return set_error(XL_ERR_LAUNCH, "xl_mlstm_chunkwise_fwd: LDS attribute failed: %s", hipGetErrorString(e));
   }
   auto main = [&](bool states_only, unsigned nwg, const MainArgs& m) -> int {
     if (states_only)
@@ -848,13 +846,9 @@ static int launch_d(const ChunkwiseArgs& A) {  // the tile: 128 rows for DQK <= 
 
 }  // namespace fused
 
-size_t chunkwise_fused_workspace(int B, int NH, int S, int DQK, int DV, int max_segments) {
+size_t chunkwise_fused_workspace(int B, int NH, int S, int DQK, int DV, int max_segments, bool pipelined) {
   const fused::Layout l = fused::layout_for(B, NH, S, DQK, DV, max_segments);
-  return max(l.total, l.prep_bytes + fused::split_bytes(B, NH, S, DQK, DV, max_segments));
-}
-
-int chunkwise_fused_segments(int B, int NH, int S, int DQK, int DV, int max_segments) {
-  return fused::layout_for(B, NH, S, DQK, DV, max_segments).P;
+  return pipelined ? l.prep_bytes + fused::split_bytes(B, NH, S, DQK, DV, max_segments) : l.total;
 }
 
 bool chunkwise_fused_supported(const ChunkwiseArgs& a, const char** why, bool pipelined) {

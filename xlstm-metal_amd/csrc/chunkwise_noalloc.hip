@@ -98,13 +98,13 @@ extern "C" int xl_mlstm_chunkwise_fwd_noalloc(const void* q, const void* k, cons
   const char* why = nullptr;
   if (!chunkwise_fused_supported(a, &why, false))
     return set_error(XL_ERR_UNSUPPORTED, "xl_mlstm_chunkwise_fwd_noalloc: fused algorithm unsupported here: %s", why);
-  const size_t need = chunkwise_fused_workspace(B, NH, S, DQK, DV, 1);
+  const size_t need = chunkwise_fused_workspace(B, NH, S, DQK, DV, 1, false);
   if (need > (size_t)XL_NOALLOC_SCRATCH_BYTES)
     return set_error(XL_ERR_UNSUPPORTED,
                      "xl_mlstm_chunkwise_fwd_noalloc: B*NH*ceil(S/64) = %lld chunks need %zu bytes of scratch, "
                      "more than the static %zu (at most %zu chunks); use xl_mlstm_chunkwise_fwd with a workspace",
                      (long long)B * NH * ((S + 63) / 64), need, (size_t)XL_NOALLOC_SCRATCH_BYTES,
-                     (size_t)XL_NOALLOC_SCRATCH_BYTES / chunkwise_fused_workspace(1, 1, 64, DQK, DV, 1));
+                     (size_t)XL_NOALLOC_SCRATCH_BYTES / chunkwise_fused_workspace(1, 1, 64, DQK, DV, 1, false));
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   DeviceState* d = nullptr;
   rc = device_state(stream, &d);
