@@ -21,3 +21,18 @@ def test_pipelined_workspace_holds_end_states_only(B, NH, S, DQK, DV, most):
     assert states <= most * one + 256
     fused, one = _segments(B, NH, S, DQK, DV, "fused")
     assert fused <= 2 * 15 * one + 512
+
+
+# Calls timed split and unsplit: one launch where the second one costs more than it saves (6 to 12 chunks), the
+# split where it was the faster (the 7B head's prompt among them)
+@pytest.mark.parametrize("B,NH,NC,DQK,DV,split", [(1, 4, 6, 256, 512, False), (1, 4, 7, 256, 512, False),
+                                                  (1, 8, 7, 256, 512, False), (2, 8, 10, 256, 512, False),
+                                                  (2, 8, 12, 256, 512, False), (1, 8, 6, 192, 384, False),
+                                                  (1, 2, 6, 32, 64, False), (2, 8, 6, 64, 128, False),
+                                                  (1, 8, 6, 96, 192, False), (1, 8, 7, 96, 192, True),
+                                                  (1, 2, 6, 128, 256, True), (1, 8, 7, 128, 256, True),
+                                                  (1, 8, 9, 256, 512, True), (1, 8, 8, 64, 128, True),
+                                                  (1, 8, 32, 256, 512, True), (2, 8, 64, 256, 512, True)])
+def test_split_where_it_is_the_faster(B, NH, NC, DQK, DV, split):
+    states, _ = _segments(B, NH, 64 * NC, DQK, DV, "pipelined")
+    assert (states > 0) == split

@@ -712,12 +712,13 @@ static int segments_for(int B, int NH, int S, int DV, int max_seg) {
 struct Split {
   int w, n0, n;
 };
-static Split pipe_split(int B, int NH, int S, int DV, int max_seg) {
+static Split pipe_split(int B, int NH, int S, int DQK, int DV, int max_seg) {
   const long long pairs = (long long)B * NH * (DV / DVT);
   const int NC = (S + L - 1) / L;
   Split best = {0, NC, 0};
   if (pairs <= 0 || pairs * 2 > kTargetWorkgroups || max_seg < 2) return best;
   constexpr float STATE = 0.55f, LAUNCH = 1.5f, START = 0.3f;
+  auto cost_of = [&](const Split& x) { return 2 * LAUNCH + START * x.w + fmaxf((float)x.n0, STATE * x.n) + x.n; };
   float cost = 0.9f * (LAUNCH + NC);  // a split has to be worth its second launch
   const int wmax = min((int)(kTargetWorkgroups / pairs), min(kMaxSegments, max_seg) - 1);
   for (int w = 2; w <= wmax; ++w) {
@@ -725,11 +726,20 @@ static Split pipe_split(int B, int NH, int S, int DV, int max_seg) {
     for (int n = max(near, 1); n <= near + 1; ++n) {
       const int n0 = max(NC - w * n, 1);
       if (n0 + (w - 1) * n >= NC) continue;  // an empty last segment
-      const float c = 2 * LAUNCH + START * w + fmaxf((float)n0, STATE * n) + n;
-      if (c < cost) cost = c, best = {w, n0, n};
+      const Split x = {w, n0, n};
+      if (cost_of(x) < cost) cost = cost_of(x), best = x;
     }
   }
-  return best;
+  if (!best.w) return best;
+  // What that model leaves out, in the same unit: the prologue of a second launch (a 256-row tile loads more, a head
+  // narrower than 128 rows zeroes the rest), chunks that run slower with w times the workgroups, the loads of a
+  // one-chunk segment, which nothing hides.  Fitted to 528 calls of 6 to 16 chunks at DQK 32 to 256 and 1 to 128
+  // (head, column tile) pairs, timed split and unsplit: without it the shortest splits were up to 17 % slower than
+  // one launch (28.0 / 24.0 us at 6 chunks of B1 NH4 DQK256 DV512, 42.7 / 38.8 at 10 of B2 NH8); with it the choice
+  // is within 1 % of the better of the two for all but 21 of them, the worst of those 9 % off.
+  const float tile = DQK > 128 ? 1.18f : fminf(1.1f, 3.f - DQK * (3.f / 128));
+  const float extra = tile + pairs * best.w / 256.f + (best.n == 1 ? 0.35f : 0.f);
+  return LAUNCH + NC - cost_of(best) > extra ? best : Split{0, NC, 0};
 }
 
 struct Layout {  // workspace: gate prep, then (split only) the end states and start states
@@ -754,13 +764,13 @@ static Layout layout_for(int B, int NH, int S, int DQK, int DV, int max_seg) {
 
 // bytes of the pipelined kernel's end states (C, n, m, total log forget gate per segment and head)
 static size_t split_bytes(int B, int NH, int S, int DQK, int DV, int max_seg) {
-  const Split sp = pipe_split(B, NH, S, DV, max_seg);
+  const Split sp = pipe_split(B, NH, S, DQK, DV, max_seg);
   return align256((size_t)sp.w * B * NH * ((size_t)DQK * DV + DQK + 2) * sizeof(float));
 }
 
 static int launch_pipe(const ChunkwiseArgs& A, int DQK, float* prep) {
   const int BNH = A.B * A.NH, NC = (A.S + L - 1) / L;
-  const Split s = pipe_split(A.B, A.NH, A.S, A.DV, A.max_segments);
+  const Split s = pipe_split(A.B, A.NH, A.S, A.DQK, A.DV, A.max_segments);
   const int strided = A.strides[2] != 0;
   auto strides = [&](int i) { return Strides{A.strides[3 * i], A.strides[3 * i + 1], (int)A.strides[3 * i + 2]}; };
   SplitArgs sp = {max(s.w, 1), s.n0, s.n, nullptr, nullptr, nullptr, nullptr};
