@@ -22,8 +22,9 @@ def test_forms(gpu_case, B, NH, S, DQK, DV, states):
     _run(B, NH, S, DQK, DV, 64, torch.bfloat16, states, states, seed=S + DQK + B)
 
 
-@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 2, 192, 256, 128), (1, 8, 64, 128, 1024), (1, 9, 64, 128, 1024)])
+@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 2, 192, 256, 128), (1, 8, 64, 128, 1024), (1, 9, 64, 128, 1024),
+                                           (1, 24, 64, 128, 1024), (1, 25, 64, 128, 1024)])
 def test_float32_row_slices(gpu_case, B, NH, S, DQK, DV):
-    """The float32 scans with 64 rows a workgroup (up to 128 workgroups of 128 rows: 4 slices of a state, exactly
-    128) and 128 (144), forward and backward."""
+    """The float32 scans with 64 rows a workgroup (up to 384 workgroups of 128 rows: 4 slices of a state, 128, 144,
+    exactly 384) and 128 (400), forward and backward."""
     _run(B, NH, S, DQK, DV, 64, torch.float32, True, True, seed=DV)

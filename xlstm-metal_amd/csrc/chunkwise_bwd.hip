@@ -2517,12 +2517,18 @@ __global__ __launch_bounds__(FV_THREADS) void bw_dvqk_bf16_kernel(
 }
 
 
-// 128-row workgroups (of both scans together in bw_scan_pair_kernel) up to which they take 64 rows each
+// 128-row workgroups of both scans of bw_scan_pair_kernel together up to which they take 64 rows each
 // instead, so that every CU has one: a scan's time then is its chain, 2.3 us a chunk at 128 rows, 1.5 at 64.
 // The whole backward with 64 / 128 rows: 128 workgroups 67 / 73 us (B2 NH8 S1024 DQK128 DV256) and 387 / 406
 // (B1 NH4 S8192 DQK256 DV512), 192 workgroups 163 / 153, 256 workgroups 722 / 667; the paired scans at 512
 // 305 / 244.
 constexpr int SCAN_FEW = 128;
+// The same for bw_scan_kernel (float32 and f16 q/k/v), whose chunk is bound by float32 MFMA: two 64-row workgroups
+// keep more of a CU's matrix cores busy than one of 128, until there are two of those per CU.  64 / 128 rows, the
+// float32 forward of 16 chunks at DQK256 DV512: 128 workgroups 93.1 / 113.1 us, 144 115.4 / 120.0, 256 143.1 /
+// 147.9, 384 209.2 / 232.5, 512 313.5 / 283.9; forward and backward in f16 at 8 chunks: 128 222.2 / 243.8, 256
+// 305.6 / 312.4, 384 402.8 / 425.0, 512 503.1 / 506.4; DQK128 DV256 alike.
+constexpr int SCAN_FEW_F32 = 384;
 
 template <typename TQ, typename TG, int L, bool REV>
 int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, const float* gp, const float* s0,
@@ -2550,9 +2556,7 @@ int launch_scan(int DQK, const TQ* X, const TQ* Y, const TG* ig, const TG* fg, c
                          Sst, nst, mst, sfin, nfin, mfin, s_init, NC, DQK, DV, nvt, qk_scale);
       return check_launch(who);
     };
-    // 64 rows where 128 would leave CUs without a workgroup: a chunk is a chain of staging, stores and MFMAs
-    // on few waves (float32 B1 NH8 S1024 DQK256 DV512: 79.6 -> 58.5 us)
-    if (DQK == 64 || BNH * nvt * (DQK / 128) <= SCAN_FEW)
+    if (DQK == 64 || BNH * nvt * (DQK / 128) <= SCAN_FEW_F32)
       return go(bw_scan_kernel<TQ, TG, L, 1, REV>, scan_smem<TQ, L>(1), DQK / 64);
     return go(bw_scan_kernel<TQ, TG, L, 2, REV>, scan_smem<TQ, L>(2), DQK / 128);
   }
