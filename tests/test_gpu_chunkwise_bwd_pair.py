@@ -28,3 +28,11 @@ def test_float32_row_slices(gpu_case, B, NH, S, DQK, DV):
     """The float32 scans with 64 rows a workgroup (up to 384 workgroups of 128 rows: 4 slices of a state, 128, 144,
     exactly 384) and 128 (400), forward and backward."""
     _run(B, NH, S, DQK, DV, 64, torch.float32, True, True, seed=DV)
+
+
+@pytest.mark.parametrize("DQK", [64, 128, 256])
+@pytest.mark.parametrize("DV", [256, 512])
+@pytest.mark.parametrize("S", [64, 1024 + 64])
+def test_gate_partials(gpu_case, DQK, DV, S):
+    """The gate pass at every count of partials that the fused path has, in one 1024-token segment and two."""
+    _run(1, 2, S, DQK, DV, 64, torch.bfloat16, False, True, seed=DQK + DV)

@@ -625,9 +625,10 @@ __global__ __launch_bounds__(BW_THREADS) void bw_dqk_kernel(const TQ* __restrict
 // each workgroup sums itself (a plain reduction over contiguous partials).
 constexpr int GSEG = 1024;
 
-// NDT, NVT: the partials per token, 0 where only known at run time.  Every load is issued before the first
-// sum (the partials of a thread's 4 tokens and 16-byte pieces of the later segments': with one load at a
-// time the pass took 25 us at B2 NH8 S4096 DQK256 DV512, so 9).
+// NDT, NVT: the partials per token.  With them every load is issued before the first sum (the partials of a
+// thread's 4 tokens and 16-byte pieces of the later segments'): B2 NH8 S4096, one load at a time / so: DQK256 DV512
+// 25 / 9.5 us; with the run-time form below / so: DQK64 DV256 7.5 / 5.0, DQK64 DV512 10.9 / 6.4, DQK128 DV512 12.6 /
+// 7.4, DQK256 DV256 13.2 / 8.2.  0: known at run time only, a token's partials one load after another.
 template <typename TG, int NDT, int NVT>
 __global__ __launch_bounds__(256) void bw_gates_kernel(const TG* __restrict__ fg, const float* __restrict__ dfp,
                                                        const float* __restrict__ dip, TG* __restrict__ di,
@@ -2570,9 +2571,17 @@ int launch_gates(const TG* fg, const float* dfp, const float* dip, void* di, voi
                        (TG*)df, S, ndt, nvt);
     return check_launch("xl_mlstm_chunkwise_bwd(gates)");
   };
-  if (ndt == 4 && nvt == 8) return go(bw_gates_kernel<TG, 4, 8>);
-  if (ndt == 2 && nvt == 4) return go(bw_gates_kernel<TG, 2, 4>);
-  return go(bw_gates_kernel<TG, 0, 0>);
+  // every head of the fused path (DQK 64, 128, 256; DV 256, 512); behind the unfused passes, whose head widths are
+  // many and whose times are several times the fused pass's, the run-time form
+  switch (nvt == 4 || nvt == 8 ? 16 * ndt + nvt : 0) {
+    case 16 + 4: return go(bw_gates_kernel<TG, 1, 4>);
+    case 16 + 8: return go(bw_gates_kernel<TG, 1, 8>);
+    case 32 + 4: return go(bw_gates_kernel<TG, 2, 4>);
+    case 32 + 8: return go(bw_gates_kernel<TG, 2, 8>);
+    case 64 + 4: return go(bw_gates_kernel<TG, 4, 4>);
+    case 64 + 8: return go(bw_gates_kernel<TG, 4, 8>);
+    default: return go(bw_gates_kernel<TG, 0, 0>);
+  }
 }
 
 template <typename TQ, typename TG, int L>
