@@ -29,3 +29,47 @@ def test_training_step_traces_with_symbolic_sizes(S, algo, states):
     assert called == ["xlstm_hip.mlstm_chunkwise.default", "xlstm_hip.mlstm_chunkwise_bwd.default"]
     q = next(n for n in gm.graph.nodes if n.op == "placeholder").meta["val"]
     assert all(not d.node.expr.is_number for d in q.shape), f"sizes fixed to the traced ones: {q.shape}"
+
+
+def _step_inputs(leaf):
+    q, k, v = (torch.randn(1, 2, d, device="cuda") for d in (64, 64, 128))
+    i, f, m = (torch.randn(1, 2, 1, device="cuda") for _ in range(3))
+    return (q, k, v, i, f), torch.randn(1, 2, 64, 128, device="cuda", requires_grad=leaf), torch.rand(1, 2, 64, device="cuda"), m
+
+
+def test_in_place_ops_move_version_counters_under_fake_tensors():
+    import xlstm_hip
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x, C, n, m = _step_inputs(False)
+        before = C._version
+        xlstm_hip.mlstm_recurrent_step_(*x, C, n, m)
+        assert C._version == before + 1
+        a, w = torch.randn(2, 16, device="cuda", dtype=torch.bfloat16), torch.ones(16, device="cuda", dtype=torch.bfloat16)
+        src, dst = torch.randn(4, device="cuda"), torch.zeros(4, device="cuda")
+        torch.ops.xlstm_hip.add_rmsnorm(a, a, w, 1e-6, [src], [dst])
+        assert dst._version == 1 and src._version == 0
+
+
+@pytest.mark.parametrize("where", ["leaf C", "computed C", "q"])
+def test_in_place_step_where_a_gradient_is_wanted(where):
+    """C may require a gradient, as a leaf too: it is updated outside autograd (its own history stays), and
+    a backward through the outputs raises."""
+    import xlstm_hip
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x, C, n, m = _step_inputs(where != "q")
+        if where == "q":
+            x[0].requires_grad_(True)
+        elif where == "computed C":
+            C = C * 1.0
+        history = C.grad_fn
+        h, (_, n1, m1) = xlstm_hip.mlstm_recurrent_step_(*x, C, n, m)
+        assert C.grad_fn is history and C._version == 1
+        assert h.grad_fn is not None and n1.grad_fn is not None and m1.grad_fn is not None
+        with pytest.raises(RuntimeError):
+            n1.grad_fn(None, torch.ones_like(n1), None)
+    with torch.no_grad(), FakeTensorMode():
+        x, C, n, m = _step_inputs(True)
+        h, _ = xlstm_hip.mlstm_recurrent_step_(*x, C, n, m)
+        assert not h.requires_grad

@@ -13,6 +13,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
 
 #include <optional>
@@ -80,11 +82,6 @@ void check_rc(int rc, const char* what) {
   TORCH_CHECK(rc != XL_ERR_WORKSPACE, what, ": ", msg, " (workspace)");
   TORCH_CHECK(rc != XL_ERR_LAUNCH, what, ": ", msg, " (launch)");
   TORCH_CHECK(false, what, ": ", msg, " (code ", rc, ")");
-}
-
-// t was written in place: autograd's version counter moves (inference tensors have none)
-void wrote(const Tensor& t) {
-  if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
 }
 
 at::TensorOptions f32_on(const Tensor& t) { return t.options().dtype(at::kFloat); }
@@ -159,9 +156,7 @@ std::tuple<Tensor, Tensor, Tensor> mlstm_step_(const Tensor& q, const Tensor& k,
   const StepShape s = step_shapes(q, k, v, i, f, c, n, m, what);
   XL_CHECK(c.scalar_type() == at::kFloat && c.is_contiguous() && ((uintptr_t)c.const_data_ptr() & 15u) == 0, what,
            "in-place C must be a contiguous, 16-byte aligned float32 tensor");
-  auto out = launch_step(q, k, v, i, f, c, n, m, c, s, eps, qk_scale, gpu, what);
-  wrote(c);
-  return out;
+  return launch_step(q, k, v, i, f, c, n, m, c, s, eps, qk_scale, gpu, what);
 }
 
 // -------------------------------------------------------- chunkwise / sequence
@@ -611,7 +606,6 @@ std::tuple<Tensor, Tensor> norm_impl(const char* what, const Tensor& x_, const T
   check_rc(xl_add_rmsnorm_fwd(ptr(x), ptr(r), ptr(w), ptr(s), ptr(y), i32(D ? x.numel() / D : 0, what), i32(D, what),
                               (float)eps, cp[0][0], cp[0][1], n[0], cp[1][0], cp[1][1], n[1], dtype_code(x, what), gpu.st),
            what);
-  for (const Tensor& t : dst) wrote(t);
   return {s, y};
 }
 
@@ -631,6 +625,76 @@ Tensor silu_mul(const Tensor& g_, const Tensor& u_) {
   const Tensor g = prep(g_), u = prep(u_), y = like(g);
   check_rc(xl_silu_mul_fwd(ptr(g), ptr(u), ptr(y), y.numel(), dtype_code(y, what), gpu.st), what);
   return y;
+}
+
+// The operators that write an argument, under autograd's bookkeeping, on fake tensors as on real ones.  What they
+// write is updated outside autograd, whatever it requires (a leaf too; its own history stays), a backward through
+// the outputs raises, and the written tensors' version counters move (inference tensors have none).
+template <typename Op, typename... Args>
+auto without_backward(const char* name, const Op& op, c10::DispatchKeySet ks, at::TensorList given, const Args&... args) {
+  bool grad = false;
+  for (const Tensor& t : given) {
+    TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(0).defined(), name, ": no forward-mode derivative");
+    grad = grad || t.requires_grad();
+  }
+  grad = grad && c10::GradMode::is_enabled();
+  auto out = [&] {
+    at::AutoDispatchBelowAutograd below;
+    return op.redispatch(ks & c10::after_autograd_keyset, args...);
+  }();
+  if (grad) {
+    const auto none = std::make_shared<torch::autograd::NotImplemented>(name);
+    none->set_next_edges(torch::autograd::collect_next_edges(given));
+    std::apply([&](const auto&... t) { (torch::autograd::set_history(t, none), ...); }, out);
+  }
+  return out;
+}
+
+template <typename Op, typename... Args>
+auto and_count(const Op& op, c10::DispatchKeySet ks, at::TensorList written, const Args&... args) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  auto out = op.redispatch(ks & c10::after_ADInplaceOrView_keyset, args...);
+  for (const Tensor& t : written)
+    if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+  return out;
+}
+
+const auto& step_inplace_op() {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("xlstm_hip::mlstm_step_", "").typed<decltype(mlstm_step_)>();
+  return op;
+}
+
+std::tuple<Tensor, Tensor, Tensor> mlstm_step__autograd(c10::DispatchKeySet ks, const Tensor& q, const Tensor& k,
+                                                        const Tensor& v, const Tensor& i, const Tensor& f, const Tensor& c,
+                                                        const Tensor& n, const Tensor& m, double eps, double qk_scale) {
+  return without_backward("xlstm_hip::mlstm_step_", step_inplace_op(), ks, {q, k, v, i, f, c, n, m}, q, k, v, i, f, c, n,
+                          m, eps, qk_scale);
+}
+
+std::tuple<Tensor, Tensor, Tensor> mlstm_step__inplace(c10::DispatchKeySet ks, const Tensor& q, const Tensor& k,
+                                                       const Tensor& v, const Tensor& i, const Tensor& f, const Tensor& c,
+                                                       const Tensor& n, const Tensor& m, double eps, double qk_scale) {
+  return and_count(step_inplace_op(), ks, {c}, q, k, v, i, f, c, n, m, eps, qk_scale);
+}
+
+const auto& add_rmsnorm_op() {
+  static const auto op =
+      c10::Dispatcher::singleton().findSchemaOrThrow("xlstm_hip::add_rmsnorm", "").typed<decltype(add_rmsnorm)>();
+  return op;
+}
+
+std::tuple<Tensor, Tensor> add_rmsnorm_autograd(c10::DispatchKeySet ks, const Tensor& x, const Tensor& r, const Tensor& w,
+                                                double eps, at::TensorList src, at::TensorList dst) {
+  std::vector<Tensor> given = {x, r, w};
+  given.insert(given.end(), src.begin(), src.end());
+  given.insert(given.end(), dst.begin(), dst.end());
+  return without_backward("xlstm_hip::add_rmsnorm", add_rmsnorm_op(), ks, given, x, r, w, eps, src, dst);
+}
+
+std::tuple<Tensor, Tensor> add_rmsnorm_inplace(c10::DispatchKeySet ks, const Tensor& x, const Tensor& r, const Tensor& w,
+                                               double eps, at::TensorList src, at::TensorList dst) {
+  return and_count(add_rmsnorm_op(), ks, dst, x, r, w, eps, src, dst);
 }
 
 }  // namespace
@@ -658,11 +722,17 @@ TORCH_LIBRARY_IMPL(xlstm_hip, CUDA, m) {
 // The chunkwise forward differentiates through its own backward; every other operator is forward-only and
 // a backward through it raises.
 #define XL_FORWARD_ONLY(m, kernel)                                                                                     \
-  for (const char* op : {"soft_cap", "mlstm_step", "mlstm_step_", "mlstm_chunkwise_bwd", "mlstm_sequence", "slstm_step", \
+  for (const char* op : {"soft_cap", "mlstm_step", "mlstm_chunkwise_bwd", "mlstm_sequence", "slstm_step",              \
                          "slstm_sequence", "causal_conv1d", "group_norm", "mh_rmsnorm_gate", "gate_proj_softcap",      \
-                         "gate_proj2_softcap", "lm_head_softcap", "rms_norm", "add_rmsnorm", "silu_mul"})              \
+                         "gate_proj2_softcap", "lm_head_softcap", "rms_norm", "silu_mul"})                             \
     m.impl(op, kernel());
 TORCH_LIBRARY_IMPL(xlstm_hip, Autograd, m) {
   m.impl("mlstm_chunkwise", mlstm_chunkwise_autograd);
+  m.impl("mlstm_step_", mlstm_step__autograd);
+  m.impl("add_rmsnorm", add_rmsnorm_autograd);
   XL_FORWARD_ONLY(m, torch::autograd::autogradNotImplementedFallback)
+}
+TORCH_LIBRARY_IMPL(xlstm_hip, ADInplaceOrView, m) {
+  m.impl("mlstm_step_", mlstm_step__inplace);
+  m.impl("add_rmsnorm", add_rmsnorm_inplace);
 }
