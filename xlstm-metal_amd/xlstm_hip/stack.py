@@ -38,6 +38,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .backend import (get_mlstm_kernel, get_mlstm_sequence_kernel, get_mlstm_step_kernel,
                       wrap_chunkwise__arbitrary_sequence_length)
@@ -99,20 +100,33 @@ CFG3_STACK = StackConfig("cfg3_xlstm7b", d_model=4096, num_blocks=32, mlstm_head
 CFG4_STACK = StackConfig("cfg4_mixed", d_model=2048, num_blocks=24, mlstm_heads=8, slstm_every=8)
 
 
-def _one_pass(x: Tensor, other: Tensor) -> bool:
-    """Whether the block's element-wise kernels (csrc/block_ops.hip) take x: GPU tensors of one 16-bit
-    dtype, rows of a multiple of 8 values, no gradient recorded (the kernels are forward-only)."""
-    return (x.device.type == "cuda" and x.dtype in (torch.bfloat16, torch.float16) and other.dtype == x.dtype
-            and x.shape[-1] % 8 == 0 and not (torch.is_grad_enabled() and (x.requires_grad or other.requires_grad)))
+def _one_pass(x: Tensor, *others: Tensor) -> bool:
+    """Whether the block's element-wise kernels (csrc/block_ops.hip) take x with these: GPU tensors of one
+    16-bit dtype, rows of a multiple of 8 values, no derivative wanted and no torch.func transform under way
+    (the kernels are forward-only)."""
+    return (x.device.type == "cuda" and x.dtype in (torch.bfloat16, torch.float16) and x.shape[-1] % 8 == 0
+            and x.shape[-1] > 0 and all(t.dtype == x.dtype for t in others)
+            and not (torch.is_grad_enabled() and (x.requires_grad or any(t.requires_grad for t in others)))
+            and forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active())
+
+
+def _plain_copy(src: Tensor, dst: Tensor) -> bool:
+    """Whether a state copy is one of float32 values in memory order, with no derivative wanted."""
+    return (src.dtype == dst.dtype == torch.float32 and src.shape == dst.shape and src.device == dst.device
+            and src.is_contiguous() and dst.is_contiguous()
+            and not (torch.is_grad_enabled() and (src.requires_grad or dst.requires_grad)))
 
 
 def _add_norm(x: Tensor, r: Optional[Tensor], norm: "_RMSNorm", copies=()):
-    """(x + r, norm(x + r)), r None: (x, norm(x)); copies: up to two (source, destination) float32 states
-    copied by the same launch."""
-    if r is not None and _one_pass(x, norm.weight):
-        return add_rmsnorm_op(x, r, norm.weight, norm.eps, [s for s, _ in copies], [d for _, d in copies])
-    for s, d in copies:
-        d.copy_(s)
+    """(x + r, norm(x + r)), r None: (x, norm(x)); copies: (source, destination) states copied along, by the
+    same launch where the kernel can."""
+    one_pass = r is not None and r.shape == x.shape and _one_pass(x, r, norm.weight)
+    along = copies if one_pass and len(copies) <= 2 and all(_plain_copy(s, d) for s, d in copies) else ()
+    if not along:
+        for s, d in copies:
+            d.copy_(s)
+    if one_pass:
+        return add_rmsnorm_op(x, r, norm.weight, norm.eps, [s for s, _ in along], [d for _, d in along])
     x = x if r is None else x + r
     return x, norm(x)
 
