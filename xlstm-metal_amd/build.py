@@ -79,16 +79,17 @@ def _compile_ops() -> str:
     return obj
 
 
-def _link_ops(obj: str) -> None:
-    import torch
-    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    tmp = OPS_LIB + ".tmp"
-    cmd = ["g++", "-shared", "-fPIC", "-o", tmp, obj, f"-L{LIBDIR}", "-lxlstm_hip", "-Wl,-rpath,$ORIGIN", f"-L{tlib}",
-           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,--no-as-needed"]
+def _link(cmd: list[str]) -> None:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{res.stderr}")
-    os.replace(tmp, OPS_LIB)
+
+
+def _link_ops(obj: str, libdir: str, out: str) -> None:
+    import torch
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _link(["g++", "-shared", "-fPIC", "-o", out, obj, f"-L{libdir}", "-lxlstm_hip", "-Wl,-rpath,$ORIGIN", f"-L{tlib}",
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,--no-as-needed"])
 
 
 def build(jobs: int | None = None, verbose: bool = True) -> str:
@@ -100,13 +101,14 @@ def build(jobs: int | None = None, verbose: bool = True) -> str:
         ops = ex.submit(_compile_ops)
         objs = list(ex.map(_compile, srcs))
         ops_obj = ops.result()
-    tmp = LIB + ".tmp"
-    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"link failed: {' '.join(cmd)}\n{res.stderr}")
-    os.replace(tmp, LIB)
-    _link_ops(ops_obj)
+    # both linked before either is replaced: a failed link leaves the pair that was there
+    new = os.path.join(BUILD, "lib")
+    os.makedirs(new, exist_ok=True)
+    lib, ops_lib = os.path.join(new, os.path.basename(LIB)), os.path.join(new, os.path.basename(OPS_LIB))
+    _link([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", lib, *objs])
+    _link_ops(ops_obj, new, ops_lib)
+    os.replace(lib, LIB)
+    os.replace(ops_lib, OPS_LIB)
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources and {OPS_LIB}")
     return LIB
