@@ -1,8 +1,12 @@
-"""The pair of libraries, built together (no GPU): a failed link leaves the old pair in place."""
+"""The pair of libraries, built and loaded together (no GPU): a failed link leaves the old pair in place, and operators
+built against another C ABI than the library beside them refuse to run instead of passing it wrong arguments."""
 
 import importlib.util
 import os
+import re
+import shutil
 import subprocess
+import sys
 
 import pytest
 
@@ -33,3 +37,25 @@ def test_failed_link_keeps_both_libraries(tmp_path, monkeypatch):
     with pytest.raises(RuntimeError, match="link failed"):
         b.build(verbose=False)
     assert [open(p).read() for p in (b.LIB, b.OPS_LIB)] == ["old", "old"]
+
+
+# python_too: Python's declarations were rebuilt with the library, the operators alone were not
+@pytest.mark.parametrize("python_too", [False, True])
+def test_operators_of_another_abi_refuse(tmp_path, python_too):
+    from xlstm_hip import _lib
+    pkg = tmp_path / "xlstm_hip"
+    shutil.copytree(os.path.join(PKG, "xlstm_hip"), pkg, ignore=shutil.ignore_patterns("*.so", "__pycache__"))
+    os.makedirs(pkg / "lib", exist_ok=True)
+    shutil.copy(_lib.OPS_PATH, pkg / "lib" / "libxlstm_torch.so")
+    stub = "".join(f"int {n}(void) {{ return {99 if n == 'xl_abi_version' else -1}; }}\n" for n in _lib.SIGNATURES)
+    (tmp_path / "stub.c").write_text(stub)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(pkg / "lib" / "libxlstm_hip.so"), str(tmp_path / "stub.c")],
+                   check=True)
+    if python_too:
+        src = (pkg / "_lib.py").read_text()
+        (pkg / "_lib.py").write_text(re.sub(r"^ABI_VERSION = \d+", "ABI_VERSION = 99", src, flags=re.M))
+    code = "import xlstm_hip; print(xlstm_hip.ops.unavailable)"
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)}, cwd=tmp_path)
+    assert out.returncode == 0, out.stderr
+    assert "ABI" in out.stdout and "build both libraries again" in out.stdout

@@ -697,9 +697,14 @@ std::tuple<Tensor, Tensor> add_rmsnorm_inplace(c10::DispatchKeySet ks, const Ten
   return and_count(add_rmsnorm_op(), ks, dst, x, r, w, eps, src, dst);
 }
 
+// The kernels below call the library with this build's argument lists: none is registered over one of another ABI
+// (xlstm_hip/_lib.py then says so in their place).
+bool abi_matches() { return xl_abi_version() == XL_ABI_VERSION; }
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(xlstm_hip, CUDA, m) {
+  if (!abi_matches()) return;
   m.impl("soft_cap", soft_cap);
   m.impl("mlstm_step", mlstm_step);
   m.impl("mlstm_step_", mlstm_step_);
@@ -727,12 +732,14 @@ TORCH_LIBRARY_IMPL(xlstm_hip, CUDA, m) {
                          "gate_proj2_softcap", "lm_head_softcap", "rms_norm", "silu_mul"})                             \
     m.impl(op, kernel());
 TORCH_LIBRARY_IMPL(xlstm_hip, Autograd, m) {
+  if (!abi_matches()) return;
   m.impl("mlstm_chunkwise", mlstm_chunkwise_autograd);
   m.impl("mlstm_step_", mlstm_step__autograd);
   m.impl("add_rmsnorm", add_rmsnorm_autograd);
   XL_FORWARD_ONLY(m, torch::autograd::autogradNotImplementedFallback)
 }
 TORCH_LIBRARY_IMPL(xlstm_hip, ADInplaceOrView, m) {
+  if (!abi_matches()) return;
   m.impl("mlstm_step_", mlstm_step__inplace);
   m.impl("add_rmsnorm", add_rmsnorm_inplace);
 }

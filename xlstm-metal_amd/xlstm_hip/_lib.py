@@ -68,12 +68,21 @@ def missing(path: str = OPS_PATH) -> str:
             "`python xlstm-metal_amd/build.py` (there is no CPU fallback)")
 
 
-def load_ops() -> bool:
-    """Loads the operator kernels; False where they have not been built (the ops then raise)."""
+def load_ops() -> str:
+    """Loads the operator kernels.  Returns "" or why they cannot run (the ops then raise it): not built, or the
+    two libraries and this file's declarations are not of one build."""
     if not (os.path.exists(OPS_PATH) and os.path.exists(LIB_PATH)):
-        return False
-    torch.ops.load_library(OPS_PATH)
-    return True
+        return missing()
+    stale = "; build both libraries again with `python xlstm-metal_amd/build.py`"
+    try:
+        load()
+        torch.ops.load_library(OPS_PATH)
+    except (RuntimeError, AttributeError, OSError) as e:
+        return f"{e}{stale}"
+    # it registers nothing over a library of another ABI (csrc/torch_ops.cpp, abi_matches)
+    if not torch._C._dispatch_has_kernel_for_dispatch_key("xlstm_hip::soft_cap", "CUDA"):
+        return f"xlstm_hip: {OPS_PATH} was built for another ABI than {LIB_PATH}{stale}"
+    return ""
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:

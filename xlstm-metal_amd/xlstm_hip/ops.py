@@ -82,9 +82,10 @@ def _no_path(name: str, reason):
 
 for _name in _SCHEMAS:
     _library.impl(_name, _no_path(_name, lambda: "tensors must be on the GPU (got cpu); there is no CPU path"), "CPU")
-if not _lib.load_ops():
+unavailable = _lib.load_ops()  # "" or why the GPU kernels cannot run
+if unavailable:
     for _name in _SCHEMAS:
-        _library.impl(_name, _no_path(_name, _lib.missing), "CUDA")
+        _library.impl(_name, _no_path(_name, lambda: unavailable), "CUDA")
 
 
 def _fake(name: str):
