@@ -1,6 +1,7 @@
 """The pair of libraries, built and loaded together (no GPU): a failed link leaves the old pair in place, and operators
 built against another C ABI than the library beside them refuse to run instead of passing it wrong arguments."""
 
+import ctypes
 import importlib.util
 import os
 import re
@@ -59,3 +60,13 @@ def test_operators_of_another_abi_refuse(tmp_path, python_too):
                          env={**os.environ, "PYTHONPATH": str(tmp_path)}, cwd=tmp_path)
     assert out.returncode == 0, out.stderr
     assert "ABI" in out.stdout and "build both libraries again" in out.stdout
+
+
+def test_constants_are_the_librarys():
+    """The padding tokens and the lm_head's limits, which the tests and the routing read, are the ones the native
+    operators use."""
+    from xlstm_hip import _lib, ops
+    lib = ctypes.CDLL(_lib.OPS_PATH)
+    assert (ops._PAD_I, ops._PAD_F) == tuple(ctypes.c_double.in_dll(lib, n).value for n in ("xl_pad_i", "xl_pad_f"))
+    assert (ops.LM_HEAD_MAX_ROWS, ops.LM_HEAD_MAX_LDS) == tuple(
+        ctypes.c_int64.in_dll(lib, n).value for n in ("xl_lm_head_max_rows", "xl_lm_head_max_lds"))

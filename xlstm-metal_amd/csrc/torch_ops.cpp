@@ -23,6 +23,15 @@
 
 #include "xlstm_hip.h"
 
+// Constants that xlstm_hip/ops.py reads: the backward's padding tokens; the most rows of lm_head_softcap and the
+// LDS bytes its staged form has for rows * (D + 8) 16-bit values.
+extern "C" {
+extern const double xl_pad_i, xl_pad_f;
+extern const int64_t xl_lm_head_max_rows, xl_lm_head_max_lds;
+const double xl_pad_i = -3.0e4, xl_pad_f = 30.0;
+const int64_t xl_lm_head_max_rows = 16, xl_lm_head_max_lds = 160 * 1024;
+}
+
 namespace {
 
 using at::Tensor;
@@ -283,10 +292,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> mlstm_chunkwise_bwd(
 // do not depend on the chunk size (tests/test_oracle_chunkwise_bw.py::test_chunk_size_invariant), so any other
 // size runs at 64, and so does a sequence that the single-pass forward took with a ragged last chunk,
 // padded to whole 64-token chunks with state-preserving tokens whose gradients are dropped: an input gate
-// of kPadI makes exp(i - m) = 0 and leaves every stabiliser alone, logsigmoid(kPadF) = -9.4e-14 makes the
+// of xl_pad_i makes exp(i - m) = 0 and leaves every stabiliser alone, logsigmoid(xl_pad_f) = -9.4e-14 makes the
 // forget factor 1 to float32 precision, so (C, n, m) and the last state's gradient pass through them
-// unchanged (ops._PAD_I, ops._PAD_F; test_state_preserving_padding).
-constexpr double kPadI = -3.0e4, kPadF = 30.0;
+// unchanged (read by ops._PAD_I, ops._PAD_F; test_state_preserving_padding).
 
 // Sizes stay symbolic from here to the backward's results: a traced training step then serves every
 // sequence length (the kernels above get plain integers from the dispatcher).
@@ -337,8 +345,8 @@ struct ChunkwiseFn : public torch::autograd::Function<ChunkwiseFn> {
     if (ragged) {
       const c10::SymInt pad = L - S % L;
       for (Tensor* t : {&q, &k, &v, &dh}) *t = at::constant_pad_nd_symint(*t, {0, 0, 0, pad});
-      i = at::constant_pad_nd_symint(i, {0, pad}, kPadI);
-      f = at::constant_pad_nd_symint(f, {0, pad}, kPadF);
+      i = at::constant_pad_nd_symint(i, {0, pad}, xl_pad_i);
+      f = at::constant_pad_nd_symint(f, {0, pad}, xl_pad_f);
     }
     auto [dq, dk, dv, di, df, dc0] = bwd.call(q, k, v, i, f, given(c0), given(n0), given(m0), dh, dcl,
                                               ctx->saved_data["qk_scale"].toDouble(), L, ctx->saved_data["eps"].toDouble());
@@ -562,7 +570,6 @@ std::tuple<Tensor, Tensor> gate_proj2_softcap(const Tensor& x_, const Tensor& w1
 
 Tensor lm_head_softcap(const Tensor& x_, const Tensor& w_, double cap) {
   const char* what = "lm_head_softcap";
-  constexpr int64_t MAX_ROWS = 16, MAX_LDS = 160 * 1024;  // ops.LM_HEAD_MAX_ROWS, LM_HEAD_MAX_LDS
   Gpu gpu(what, {&x_, &w_});
   XL_CHECK(x_.dim() >= 1 && w_.dim() == 2 && w_.size(1) == x_.size(-1), what,
            "weight must be (V, D) with D = x.shape[-1], got ", w_.sizes(), " for x ", x_.sizes());
@@ -570,9 +577,9 @@ Tensor lm_head_softcap(const Tensor& x_, const Tensor& w_, double cap) {
   const int64_t V = w_.size(0), D = w_.size(1);
   std::vector<int64_t> shape;
   const int64_t M = rows_of(x_, V, shape);
-  XL_CHECK(M <= MAX_ROWS, what, M, " rows (at most ", MAX_ROWS,
+  XL_CHECK(M <= xl_lm_head_max_rows, what, M, " rows (at most ", xl_lm_head_max_rows,
            "; logits of every position are a GEMM: use the Linear and soft_cap)");
-  XL_CHECK(M * (D + 8) * 2 <= MAX_LDS, what, M, " rows of D=", D, " exceed the kernel's LDS staging");
+  XL_CHECK(M * (D + 8) * 2 <= xl_lm_head_max_lds, what, M, " rows of D=", D, " exceed the kernel's LDS staging");
   const Tensor x = prep(x_), w = prep(w_), y = at::empty(shape, x.options());
   check_rc(xl_lm_head_softcap_fwd(ptr(x), ptr(w), ptr(y), i32(M, what), i32(D, what), i32(V, what), (float)cap,
                                   dtype_code(x, what), gpu.st),

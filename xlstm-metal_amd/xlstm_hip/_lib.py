@@ -85,6 +85,11 @@ def load_ops() -> str:
     return ""
 
 
+def ops_constant(name: str, ctype):
+    """A constant of the operator library (zero where it is not built)."""
+    return ctype.in_dll(ctypes.CDLL(OPS_PATH), name).value if os.path.exists(OPS_PATH) else ctype().value
+
+
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Loads the library once and declares every signature; raises if absent."""
     global _lib

@@ -10,6 +10,7 @@ op raises.
 
 from __future__ import annotations
 
+import ctypes
 import warnings
 
 import torch
@@ -228,10 +229,11 @@ add_rmsnorm_op = torch.ops.xlstm_hip.add_rmsnorm.default
 silu_mul_op = torch.ops.xlstm_hip.silu_mul.default
 
 CONV_ACTS = {None: 0, "silu": 1}
-LM_HEAD_MAX_ROWS = 16
-LM_HEAD_MAX_LDS = 160 * 1024  # the kernel stages rows * (D + 8) 16-bit values in LDS
-# the backward's padding tokens (csrc/torch_ops.cpp: kPadI, kPadF)
-_PAD_I, _PAD_F = -3.0e4, 30.0
+# csrc/torch_ops.cpp's own: the most rows of lm_head_softcap and the LDS of its staging, and the input and
+# forget gate of the tokens that the backward pads a ragged sequence with
+LM_HEAD_MAX_ROWS = _lib.ops_constant("xl_lm_head_max_rows", ctypes.c_int64)
+LM_HEAD_MAX_LDS = _lib.ops_constant("xl_lm_head_max_lds", ctypes.c_int64)
+_PAD_I, _PAD_F = (_lib.ops_constant(_name, ctypes.c_double) for _name in ("xl_pad_i", "xl_pad_f"))
 
 
 def state_views(st: Tensor, B: int, NH: int, H: int) -> tuple[Tensor, Tensor, Tensor]:
