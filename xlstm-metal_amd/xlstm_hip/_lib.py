@@ -120,31 +120,3 @@ def check(rc: int, what: str) -> None:
         if rc == -2:
             raise NotImplementedError(f"{what}: {msg} ({kind})")
         raise RuntimeError(f"{what}: {msg} ({kind})")
-
-
-def dtype_code(t: torch.Tensor, what: str) -> int:
-    try:
-        return XL_DTYPE[t.dtype]
-    except KeyError:
-        raise ValueError(f"{what}: unsupported dtype {t.dtype} (float32, bfloat16, float16)") from None
-
-
-def ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
-
-
-def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
-def require_gpu(*tensors: torch.Tensor | None, what: str) -> None:
-    dev = None
-    for t in tensors:
-        if t is None:
-            continue
-        if t.device.type != "cuda":
-            raise RuntimeError(f"{what}: tensors must be on the GPU (got {t.device}); there is no CPU path")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"{what}: tensors on different devices ({dev} vs {t.device})")
