@@ -107,22 +107,20 @@ def wrap_chunkwise__arbitrary_sequence_length(mlstm_chunkwise_kernel, mlstm_sequ
         sizes.append(cs)
         cs //= 2
     dev = k.device
-    if S > 1 and mlstm_chunkwise_kernel in (mlstm_chunkwise__native_autograd, mlstm_chunkwise__native_custbw) \
-            and (c_initial is None) == (n_initial is None) == (m_initial is None) and _fused_takes_any_length(q, k, v):
-        # the single-pass kernel runs 64-token chunks whatever chunk_size names (the forward is
-        # chunk-size invariant), so it is called with the size its support was checked for; without
-        # initial states it starts from zeros by itself
-        h_out, last = mlstm_chunkwise_kernel(
-            q=q, k=k, v=v, f=f, i=i, c_initial=c_initial, n_initial=n_initial, m_initial=m_initial, chunk_size=64,
-            return_last_states=True, eps=eps, algo="pipelined")
-        return (h_out, last) if return_last_states else h_out
-    c_state = c_initial if c_initial is not None else torch.zeros(B, NH, DHQK, DHHV, device=dev, dtype=torch.float32)
-    n_state = n_initial if n_initial is not None else torch.zeros(B, NH, DHQK, device=dev, dtype=torch.float32)
-    m_state = m_initial if m_initial is not None else torch.zeros(B, NH, 1, device=dev, dtype=torch.float32)
-    if S > 1 and mlstm_chunkwise_kernel in (mlstm_chunkwise__native_autograd, mlstm_chunkwise__native_custbw) \
-            and _fused_takes_any_length(q, k, v):
-        # the fused kernel runs 64-token chunks whatever chunk_size names (the forward is
-        # chunk-size invariant), so it is called with the size its support was checked for
+    c_state, n_state, m_state = c_initial, n_initial, m_initial
+    single_pass = S > 1 and mlstm_chunkwise_kernel in (
+        mlstm_chunkwise__native_autograd, mlstm_chunkwise__native_custbw) and _fused_takes_any_length(q, k, v)
+    if not single_pass or any(t is not None for t in (c_state, n_state, m_state)):
+        # (the single-pass kernel starts from zeros by itself where none is given)
+        if c_state is None:
+            c_state = torch.zeros(B, NH, DHQK, DHHV, device=dev, dtype=torch.float32)
+        if n_state is None:
+            n_state = torch.zeros(B, NH, DHQK, device=dev, dtype=torch.float32)
+        if m_state is None:
+            m_state = torch.zeros(B, NH, 1, device=dev, dtype=torch.float32)
+    if single_pass:
+        # it runs 64-token chunks whatever chunk_size names (the forward is chunk-size invariant), so
+        # it is called with the size its support was checked for
         h_out, (c_state, n_state, m_state) = mlstm_chunkwise_kernel(
             q=q, k=k, v=v, f=f, i=i, c_initial=c_state, n_initial=n_state, m_initial=m_state, chunk_size=64,
             return_last_states=True, eps=eps, algo="pipelined")
