@@ -109,6 +109,31 @@ def test_chunkwise_rejects_bad_args(lib):
     assert lib.xl_mlstm_chunkwise_workspace_size(1, 8, 250, 256, 512, 64, 0, 1) == 0
 
 
+def test_chunkwise_strided_rejects_bad_args(lib):
+    f = lib.xl_mlstm_chunkwise_fwd_strided
+    p = ctypes.c_void_p(256)  # never dereferenced: validation fails first
+
+    def call(strides=(0, 256, 2048, 0, 256, 2048, 0, 512, 4096), algo=3, dtype=1, null=False):
+        s = None if null else (ctypes.c_int64 * 9)(*strides)
+        return f(p, p, p, s, p, p, None, None, None, p, None, None, None, 1, 8, 256, 256, 512, 64, 0.0625, 1e-6, dtype,
+                 dtype, algo, None, 0, None)
+
+    assert call() == -3 and b"workspace" in lib.xl_last_error()  # strides accepted
+    assert call(null=True) == -1 and b"strides" in lib.xl_last_error()
+    good = [0, 256, 2048, 0, 256, 2048, 0, 512, 4096]
+    for at, bad in ((0, 12), (1, 252), (2, 2052), (4, -8), (6, -8), (2, 248), (5, 248), (8, 504), (8, (1 << 22) + 8)):
+        s = list(good)
+        s[at] = bad  # no multiple of 8, negative, rows that overlap, rows too far apart
+        assert call(s) == -1 and b"strides" in lib.xl_last_error(), (at, bad)
+    s = list(good)
+    s[8] = 1 << 22
+    assert call(s) == -3
+    assert call(algo=1) == -2 and b"pipelined" in lib.xl_last_error()
+    assert call(algo=2) == -2
+    assert call(dtype=0) == -2  # float32: no single-pass kernel
+    assert call(dtype=0, algo=0) == -2
+
+
 def test_chunkwise_bwd_rejects_bad_args(lib):
     f = lib.xl_mlstm_chunkwise_bwd
     p, mis = ctypes.c_void_p(256), ctypes.c_void_p(264)

@@ -36,3 +36,11 @@ def test_pipelined_workspace_holds_end_states_only(B, NH, S, DQK, DV, most):
 def test_split_where_it_is_the_faster(B, NH, NC, DQK, DV, split):
     states, _ = _segments(B, NH, 64 * NC, DQK, DV, "pipelined")
     assert (states > 0) == split
+
+
+# the fewest chunks that split, 8 heads: one fewer runs in one launch
+@pytest.mark.parametrize("DQK,DV,first", [(32, 64, 7), (64, 128, 8), (96, 192, 7), (128, 256, 6), (192, 384, 8),
+                                          (256, 512, 8)])
+def test_first_split(DQK, DV, first):
+    assert [_segments(1, 8, 64 * NC, DQK, DV, "pipelined")[0] > 0 for NC in range(1, 20)] == [
+        NC >= first for NC in range(1, 20)]

@@ -79,7 +79,7 @@ def test_gate_pair(gpu_case, B, S, D, G1, G2, heads_first, cap_in_dtype):
 
 def test_stack_decode_matches_modules(gpu_case):
     """decode_step with the one-pass kernels against the same blocks run through torch's own norms and
-    SwiGLU (bit for bit: a norm's last bit may move, so rows are compared to 1 % of the logits' scale)."""
+    SwiGLU: the last bit of a norm may move and travels through the blocks, so to 1 % of the logits' scale."""
     import xlstm_hip.stack as st
     cfg = st.StackConfig("small", d_model=512, num_blocks=4, mlstm_heads=4, slstm_every=4, vocab=1000)
     model = st.xLSTMStack.random(cfg, dev(), seed=3)

@@ -2,7 +2,10 @@
 
 The strided call must be bit-equal to the call on contiguous copies (the same kernel, other addresses), over
 head widths, ragged lengths, batches, the sequence split, f16, initial states, and views whose rows cannot be
-read in place (odd row strides, an offset base, expanded rows), which take the copy."""
+read in place (odd row strides, an offset base), which take the copy; the C entry point itself against the contiguous
+one, and the operator's memory, which shows whether it copied."""
+
+import ctypes
 
 import pytest
 import torch
@@ -33,7 +36,7 @@ def _views(B, NH, S, DQK, DV, dtype, layout, seed):
     q, k, v = out
     i = torch.randn(B, NH, S, generator=g).to(dtype).to(dev())
     f = (torch.randn(B, NH, S, generator=g) + 3).to(dtype).to(dev())
-    return q / DQK ** 0.5 if layout == "plain_q" else q, k, v, i, f
+    return q, k, v, i, f
 
 
 @pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 8, 100, 256, 512), (2, 4, 1000, 128, 256), (3, 2, 65, 96, 192), (1, 2, 1, 64, 64),
@@ -47,6 +50,62 @@ def test_strided_equals_contiguous(gpu_case, B, NH, S, DQK, DV, dtype, layout):
     want = xlstm_hip.mlstm_chunkwise(*(t.contiguous() for t in x), return_last_states=True, algo="pipelined")
     for a, b in zip((got[0], *got[1]), (want[0], *want[1])):
         assert torch.equal(a, b)
+
+
+def _strides(t):
+    return [t.stride(0) if t.size(0) > 1 else 0, t.stride(1) if t.size(1) > 1 else 0, t.stride(2)]
+
+
+@pytest.mark.parametrize("B,NH,S,DQK,DV", [(1, 8, 100, 256, 512), (2, 4, 1000, 128, 256), (3, 2, 65, 96, 192)])
+@pytest.mark.parametrize("layout", ["projection", "packed", "expanded"])
+def test_strided_entry_point(gpu_case, B, NH, S, DQK, DV, layout):
+    from xlstm_hip import _lib
+    lib = _lib.load()
+    q, k, v, i, f = _views(B, NH, S, DQK, DV, torch.bfloat16, layout, S)
+    ws_bytes = lib.xl_mlstm_chunkwise_workspace_size(B, NH, S, DQK, DV, 64, 1, 3)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def run(strided):
+        x = [t if strided else t.contiguous() for t in (q, k, v)]
+        out = [torch.empty(s, dtype=d, device=dev()) for s, d in (
+            ((B, NH, S, DV), torch.bfloat16), ((B, NH, DQK, DV), torch.float32), ((B, NH, DQK), torch.float32),
+            ((B, NH), torch.float32))]
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev())
+        rest = (i.data_ptr(), f.data_ptr(), None, None, None, *(t.data_ptr() for t in out), B, NH, S, DQK, DV, 64,
+                DQK ** -0.5, 1e-6, 1, 1, 3, ws.data_ptr(), ws_bytes, st)
+        if strided:
+            strides = (ctypes.c_int64 * 9)(*[s for t in x for s in _strides(t)])
+            rc = lib.xl_mlstm_chunkwise_fwd_strided(*(t.data_ptr() for t in x), strides, *rest)
+        else:
+            rc = lib.xl_mlstm_chunkwise_fwd(*(t.data_ptr() for t in x), *rest)
+        _lib.check(rc, "strided" if strided else "contiguous")
+        torch.cuda.synchronize()
+        return out
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layout,copies", [("projection", False), ("packed", False), ("expanded", False),
+                                           ("odd_rows", True), ("offset", True)])
+def test_operator_reads_in_place(gpu_case, layout, copies):
+    """The most memory a call holds: that of the contiguous call where it reads the views in place, three copies
+    more where it cannot."""
+    import xlstm_hip
+    x = _views(2, 4, 1000, 128, 256, torch.bfloat16, layout, 3)
+
+    def peak(x):
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        xlstm_hip.mlstm_chunkwise(*x, algo="pipelined")
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - base
+
+    plain = tuple(t.contiguous() for t in x)
+    peak(plain)
+    more = peak(x) - peak(plain)
+    assert more == (sum(t.numel() * 2 for t in plain[:3]) if copies else 0)
 
 
 def test_strided_with_states_and_backend(gpu_case):

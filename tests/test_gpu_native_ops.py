@@ -55,6 +55,21 @@ def test_compiled(gpu_case):
     assert _equal(got, _grads(fn, x))
 
 
+def test_compiled_once_for_every_length(gpu_case):
+    import xlstm_hip
+    from torch._dynamo.testing import CompileCounterWithBackend
+    count = CompileCounterWithBackend("aot_eager")
+
+    def fn(q, k, v, i, f):
+        return xlstm_hip.mlstm_chunkwise(q * 1.0, k, v, i, f)
+
+    compiled = torch.compile(fn, backend=count, fullgraph=True, dynamic=True)
+    for S in (192, 320, 448):  # (128 and 256 are head widths, which tracing would tie the length to)
+        x = _x(S, seed=S, grad=True)
+        assert _equal(_grads(compiled, x), _grads(fn, x))
+    assert count.frame_count == 1
+
+
 def test_refused(gpu_case):
     import xlstm_hip
     x = torch.randn(8, 16, device=dev(), requires_grad=True)
