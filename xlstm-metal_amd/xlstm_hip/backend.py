@@ -110,7 +110,7 @@ def wrap_chunkwise__arbitrary_sequence_length(mlstm_chunkwise_kernel, mlstm_sequ
     c_state, n_state, m_state = c_initial, n_initial, m_initial
     single_pass = S > 1 and mlstm_chunkwise_kernel in (
         mlstm_chunkwise__native_autograd, mlstm_chunkwise__native_custbw) and _fused_takes_any_length(q, k, v)
-    if not single_pass or any(t is not None for t in (c_state, n_state, m_state)):
+    if not single_pass or c_state is not None or n_state is not None or m_state is not None:
         # (the single-pass kernel starts from zeros by itself where none is given)
         if c_state is None:
             c_state = torch.zeros(B, NH, DHQK, DHHV, device=dev, dtype=torch.float32)
