@@ -116,9 +116,10 @@ int xl_mlstm_step_copy_ceiling(const float* c_old, float* c_new, int B, int NH, 
  * DQK 32, 64, 96, 128, 192 or 256), and DV % 64 == 0, any S >= 1 is accepted: the kernel runs 64-token chunks and a ragged last chunk
  * (the forward is chunk-size invariant, so L only names the reference's
  * chunking there).
- * workspace: xl_mlstm_chunkwise_workspace_size(...) bytes, 256-byte aligned
- * (fused algorithm: the per-chunk gate prep, 1280 bytes per 64 tokens of
- * every head; two-pass algorithm: the chunk-entry states and the states
+ * workspace: xl_mlstm_chunkwise_workspace_size(...) bytes of the call's own arguments, algo
+ * included, 256-byte aligned (single-pass algorithms: the per-chunk gate prep, 1280 bytes per 64
+ * tokens of every head, and, where few heads make a schedule split the sequence, its segments'
+ * states; two-pass algorithm: the chunk-entry states and the states
  * pass's gate prefix, 784 bytes per chunk).  q, k, v, h, c0,
  * n0, c_last and n_last 16-byte aligned (XL_ERR_INVALID_ARG otherwise).
  */
