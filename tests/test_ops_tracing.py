@@ -73,3 +73,18 @@ def test_in_place_step_where_a_gradient_is_wanted(where):
         x, C, n, m = _step_inputs(True)
         h, _ = xlstm_hip.mlstm_recurrent_step_(*x, C, n, m)
         assert not h.requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_backend_traces_with_symbolic_sizes(dtype):
+    """The any-length wrapper looks up whether the head's widths run in one call: they are taken as numbers, the
+    length is not."""
+    import xlstm_hip
+    backend = xlstm_hip.mLSTMBackend(xlstm_hip.mLSTMBackendConfig(mode="inference"))
+    x = [t.to(dtype) for t in (torch.randn(2, 3, 100, 64), torch.randn(2, 3, 100, 64), torch.randn(2, 3, 100, 128),
+                               torch.randn(2, 3, 100), torch.randn(2, 3, 100))]
+    gm = make_fx(lambda *x: backend(*x), tracing_mode="symbolic")(*x)
+    called = [str(n.target) for n in gm.graph.nodes if "xlstm_hip" in str(n.target)]
+    assert called.count("xlstm_hip.mlstm_chunkwise.default") == (1 if dtype == torch.bfloat16 else 2)
+    q = next(n for n in gm.graph.nodes if n.op == "placeholder").meta["val"]
+    assert all(not d.node.expr.is_number for d in q.shape[:3])

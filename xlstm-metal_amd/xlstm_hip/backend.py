@@ -79,7 +79,7 @@ def _fused_takes_any_length(q, k, v) -> bool:
     ragged last chunk)."""
     if not (q.dtype == k.dtype == v.dtype and q.dtype in (torch.bfloat16, torch.float16)):
         return False
-    return _pipelined_heads(q.shape[-1], v.shape[-1], q.dtype)
+    return _pipelined_heads(int(q.shape[-1]), int(v.shape[-1]), q.dtype)  # (a traced size is no cache key)
 
 
 @lru_cache(maxsize=64)
