@@ -6,7 +6,7 @@
     python bench.py --summarize-trace TRACE_DIR              (no GPU: per-kernel durations of a kernel trace)
 
 Prints ONE JSON line.  Headline (`value`): chunkwise mLSTM prefill tokens/s
-at BASELINE config 2 (bf16 q/k/v/gates, float32 states, B4 NH8 S8192 DQK256
+at the 7B head shape (config 2: bf16 q/k/v/gates, float32 states, B4 NH8 S8192 DQK256
 DV512, L=64, last states returned).  One step = one `mlstm_chunkwise` call
 over the whole batch (B*S = 32768 tokens) with inputs resident in HBM; L2 and
 the 256 MB Infinity Cache are flushed (512 MB write) before every timed call,
@@ -741,7 +741,7 @@ def bench_arbitrary_length(args, dev):
 
 
 def bench_stack(args, dev, which):
-    """BASELINE config 3 or 4 end to end on the random-init stack (xlstm_hip.stack): prefill tokens/s
+    """Config 3 (xLSTM-7B shapes) or 4 (mixed stack) end to end on the random-init stack (xlstm_hip.stack): prefill tokens/s
     of the whole prompt (B x S tokens through every block, the final norm, the lm_head and the logit
     soft-cap of the last position) and greedy-decode tokens/s (one HIP-graph replay per token: every
     block's step kernels, the lm_head, the soft-cap and the argmax), both timed with HIP events."""
@@ -984,7 +984,7 @@ def _blas() -> str:
 
 
 def bench_cfg0(args, dev):
-    """BASELINE config 0 on the GPU: one float32 mlstm_chunkwise call (B1 NH8 S256 DQK256 DV512, L 64,
+    """Config 0 on the GPU: one float32 mlstm_chunkwise call (B1 NH8 S256 DQK256 DV512, L 64,
     last states returned): the two-pass algorithm, states on float32 MFMA, outputs on bf16 MFMA in the
     three-product form; replayed from a HIP graph, HIP events."""
     import xlstm_hip

@@ -1,4 +1,4 @@
-"""Random-init xLSTM stacks of BASELINE configs 3 and 4: the harness that runs the path's ops inside
+"""Random-init xLSTM stacks at the 7B and the mixed model's shapes (configs 3 and 4 below): the harness that runs the path's ops inside
 a whole model, for the end-to-end tests and the tokens/s figures.
 
 The block order is the reference's (paths relative to its root, ``TN`` = ``xlstm_metal/
@@ -93,9 +93,9 @@ class StackConfig:
         return self.slstm_every > 0 and (block + 1) % self.slstm_every == 0
 
 
-# xLSTM-7B shapes, 32 mLSTM blocks, d 4096, 8 heads (DQK 256, DV 512), FFN 10944
+# config 3: xLSTM-7B shapes, 32 mLSTM blocks, d 4096, 8 heads (DQK 256, DV 512), FFN 10944
 CFG3_STACK = StackConfig("cfg3_xlstm7b", d_model=4096, num_blocks=32, mlstm_heads=8)
-# d 2048, 24 blocks, mLSTM:sLSTM 7:1 (blocks 8, 16, 24 are sLSTM), mLSTM 8 heads
+# config 4: d 2048, 24 blocks, mLSTM:sLSTM 7:1 (blocks 8, 16, 24 are sLSTM), mLSTM 8 heads
 # (DQK 128, DV 256), sLSTM 4 heads of 512 with a causal conv of kernel 4
 CFG4_STACK = StackConfig("cfg4_mixed", d_model=2048, num_blocks=24, mlstm_heads=8, slstm_every=8)
 

@@ -1,6 +1,6 @@
 """Synthetic workloads of the benchmark configurations (seeded, CPU-drawn).
 
-Shapes and distributions are BASELINE's configs; draws use
+Shapes and distributions are the benchmark's configurations; draws use
 ``torch.Generator('cpu').manual_seed(seed)`` in the order q, k, v, i, f (then
 C, n, m), in float32, then cast.  Seeds: cfg0 -> 0, cfg1 -> 1, cfg2 -> 2,
 cfg4 (the sLSTM layer) -> 4.
