@@ -62,6 +62,19 @@ def test_operators_of_another_abi_refuse(tmp_path, python_too):
     assert "ABI" in out.stdout and "build both libraries again" in out.stdout
 
 
+def test_operators_without_their_library(tmp_path):
+    """Half a build imports, and every op says what to do."""
+    from xlstm_hip import _lib
+    pkg = tmp_path / "xlstm_hip"
+    shutil.copytree(os.path.join(PKG, "xlstm_hip"), pkg, ignore=shutil.ignore_patterns("*.so", "__pycache__"))
+    os.makedirs(pkg / "lib", exist_ok=True)
+    shutil.copy(_lib.OPS_PATH, pkg / "lib" / "libxlstm_torch.so")
+    out = subprocess.run([sys.executable, "-c", "import xlstm_hip; print(xlstm_hip.ops.unavailable)"], capture_output=True,
+                         text=True, timeout=120, env={**os.environ, "PYTHONPATH": str(tmp_path)}, cwd=tmp_path)
+    assert out.returncode == 0, out.stderr
+    assert "build it with" in out.stdout
+
+
 def test_constants_are_the_librarys():
     """The padding tokens and the lm_head's limits, which the tests and the routing read, are the ones the native
     operators use."""

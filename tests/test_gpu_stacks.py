@@ -1,5 +1,5 @@
-"""The 7B and the mixed stack (configs 3 and 4 of xlstm_hip.stack) on the GPU: the path's kernels at the stacks' full shapes, and the
-random-init stacks end to end (xlstm_hip.stack).
+"""The 7B and the mixed stack (configs 3 and 4 of xlstm_hip.stack) on the GPU: the path's kernels at the stacks' full
+shapes, and the random-init stacks end to end (xlstm_hip.stack).
 
 * config 3 (xLSTM-7B shapes): the mLSTM layer's prefill at B1 NH8 S2048 DQK256 DV512 bf16 on the
   q, k, v and gates a random-init block projects from a random input, against the oracle on the

@@ -86,8 +86,12 @@ def load_ops() -> str:
 
 
 def ops_constant(name: str, ctype):
-    """A constant of the operator library (zero where it is not built)."""
-    return ctype.in_dll(ctypes.CDLL(OPS_PATH), name).value if os.path.exists(OPS_PATH) else ctype().value
+    """A constant of the operator library, which load_ops has loaded."""
+    try:
+        return ctype.in_dll(ctypes.CDLL(OPS_PATH), name).value
+    except ValueError as e:
+        raise RuntimeError(f"xlstm_hip: {OPS_PATH} is of an older build ({e}); build again with "
+                           "`python xlstm-metal_amd/build.py`") from None
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:

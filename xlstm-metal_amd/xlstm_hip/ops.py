@@ -229,11 +229,12 @@ add_rmsnorm_op = torch.ops.xlstm_hip.add_rmsnorm.default
 silu_mul_op = torch.ops.xlstm_hip.silu_mul.default
 
 CONV_ACTS = {None: 0, "silu": 1}
-# csrc/torch_ops.cpp's own: the most rows of lm_head_softcap and the LDS of its staging, and the input and
-# forget gate of the tokens that the backward pads a ragged sequence with
-LM_HEAD_MAX_ROWS = _lib.ops_constant("xl_lm_head_max_rows", ctypes.c_int64)
-LM_HEAD_MAX_LDS = _lib.ops_constant("xl_lm_head_max_lds", ctypes.c_int64)
-_PAD_I, _PAD_F = (_lib.ops_constant(_name, ctypes.c_double) for _name in ("xl_pad_i", "xl_pad_f"))
+# csrc/torch_ops.cpp's own (0 where no kernel can run): the most rows of lm_head_softcap and the LDS of its
+# staging, and the input and forget gate of the tokens that the backward pads a ragged sequence with
+LM_HEAD_MAX_ROWS, LM_HEAD_MAX_LDS, _PAD_I, _PAD_F = (
+    ctype().value if unavailable else _lib.ops_constant(_name, ctype)
+    for _name, ctype in (("xl_lm_head_max_rows", ctypes.c_int64), ("xl_lm_head_max_lds", ctypes.c_int64),
+                         ("xl_pad_i", ctypes.c_double), ("xl_pad_f", ctypes.c_double)))
 
 
 def state_views(st: Tensor, B: int, NH: int, H: int) -> tuple[Tensor, Tensor, Tensor]:

@@ -1,5 +1,5 @@
-"""Random-init xLSTM stacks at the 7B and the mixed model's shapes (configs 3 and 4 below): the harness that runs the path's ops inside
-a whole model, for the end-to-end tests and the tokens/s figures.
+"""Random-init xLSTM stacks at the 7B and the mixed model's shapes (configs 3 and 4 below): the harness that
+runs the path's ops inside a whole model, for the end-to-end tests and the tokens/s figures.
 
 The block order is the reference's (paths relative to its root, ``TN`` = ``xlstm_metal/
 torch_native``):
