@@ -42,6 +42,20 @@ def test_add_rmsnorm(gpu_case, M, D, dtype, residual):
     assert float(((y.double() - want).abs() - _ulp(want, dtype)).max()) <= 0
 
 
+def test_longest_state_copy(gpu_case):
+    """A copy of 2^31 - 1 values, the most an int names, by a grid whose stride takes the index past it: whole, and
+    nothing beside it."""
+    from xlstm_hip.ops import add_rmsnorm_op
+    n = 2 ** 31 - 1
+    src = torch.full((n,), 2.0, device=dev())
+    src[-1] = 3.0
+    whole = torch.zeros(n + 64, device=dev())
+    x, w = torch.ones(4096, 8, dtype=torch.bfloat16, device=dev()), torch.ones(8, dtype=torch.bfloat16, device=dev())
+    add_rmsnorm_op(x, x, w, 1e-6, [src], [whole[:n]])
+    assert float(whole[n - 1]) == 3.0 and not whole[n:].any()
+    assert float(whole[:n - 1].min()) == float(whole[:n - 1].max()) == 2.0
+
+
 @pytest.mark.parametrize("shape", [(1, 8), (3, 5504), (4100, 2752)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_silu_mul(gpu_case, shape, dtype):

@@ -119,7 +119,8 @@ __global__ __launch_bounds__(BO_BLOCK) void add_rmsnorm_kernel(const T* __restri
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c)
-    for (int e = blockIdx.x * BO_BLOCK + tid; e < cp.n[c]; e += gridDim.x * BO_BLOCK) cp.dst[c][e] = cp.src[c][e];
+    for (int64_t e = (int64_t)blockIdx.x * BO_BLOCK + tid; e < cp.n[c]; e += (int64_t)gridDim.x * BO_BLOCK)
+      cp.dst[c][e] = cp.src[c][e];
 }
 
 template <typename T>

@@ -113,7 +113,7 @@ def _one_pass(x: Tensor, *others: Tensor) -> bool:
 def _plain_copy(src: Tensor, dst: Tensor) -> bool:
     """Whether a state copy is one of float32 values in memory order, with no derivative wanted."""
     return (src.dtype == dst.dtype == torch.float32 and src.shape == dst.shape and src.device == dst.device
-            and src.is_contiguous() and dst.is_contiguous()
+            and src.is_contiguous() and dst.is_contiguous() and src.numel() < 2 ** 31
             and not (torch.is_grad_enabled() and (src.requires_grad or dst.requires_grad)))
 
 
